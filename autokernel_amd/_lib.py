@@ -41,6 +41,9 @@ SIGNATURES: dict[str, list] = {
     "ak_cross_entropy_noalloc": [_i, _p, _p, _p, _i64, _i64, _i64, _p],
     "ak_reduce_sum": [_i, _p, _p, _i64, _i64, _i64, _p],
     "ak_reduce_max": [_i, _p, _p, _i64, _i64, _i64, _p],
+    "ak_reduce_workspace_bytes": [_i, _i64, _i64, _i64],
+    "ak_reduce_sum_ws": [_i, _p, _p, _i64, _i64, _i64, _p, _i64, _p],
+    "ak_reduce_max_ws": [_i, _p, _p, _i64, _i64, _i64, _p, _i64, _p],
     "ak_gemm": [_i, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i, _p],
     "ak_gemm_batched": [_i, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _p],
     "ak_gemm_residual": [_i, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i, _p],
@@ -57,7 +60,7 @@ SIGNATURES: dict[str, list] = {
                           _pi64, _pi64, _pi64, _pi64, _i, _f, _p],
 }
 _STR_FUNCS = ("ak_version", "ak_status_string", "ak_last_hip_error_string")
-_I64_FUNCS = ("ak_gemm_workspace_bytes",)  # return int64_t instead of a status
+_I64_FUNCS = ("ak_gemm_workspace_bytes", "ak_reduce_workspace_bytes")  # return int64_t instead of a status
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

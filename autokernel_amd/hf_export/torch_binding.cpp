@@ -7,6 +7,7 @@
 
 #include <algorithm>
 
+#include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
@@ -173,10 +174,17 @@ static void reduce_common(at::Tensor& y, const at::Tensor& x, int64_t outer, int
   TORCH_CHECK(y.numel() == outer * inner, op, ": y has ", y.numel(), " elements, expected ", outer * inner);
   const c10::DeviceGuard g(x.device());
   const int code = dtype_code(x, op);
+  // fp32 partial sums of row slices (long reductions over a dim other than the last)
+  const int64_t bytes = ak_reduce_workspace_bytes(code, outer, reduce, inner);
+  at::Tensor ws;
+  if (bytes > 0) ws = at::empty({bytes / 4}, x.options().dtype(at::kFloat));
+  void* wp = bytes > 0 ? ws.data_ptr() : nullptr;
   if (is_max)
-    check_status(ak_reduce_max(code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, stream_of(x)), "ak_reduce_max");
+    check_status(ak_reduce_max_ws(code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, wp, bytes, stream_of(x)),
+                 "ak_reduce_max_ws");
   else
-    check_status(ak_reduce_sum(code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, stream_of(x)), "ak_reduce_sum");
+    check_status(ak_reduce_sum_ws(code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, wp, bytes, stream_of(x)),
+                 "ak_reduce_sum_ws");
 }
 
 void ak_op_reduce_sum(at::Tensor& y, const at::Tensor& x, int64_t outer, int64_t reduce, int64_t inner) {

@@ -67,14 +67,29 @@ def cross_entropy(out: torch.Tensor, row_loss: torch.Tensor, logits: torch.Tenso
          shape=tuple(logits.shape), dtype=logits.dtype)
 
 
+@functools.lru_cache(maxsize=1024)
+def _reduce_workspace_bytes(dtype: int, outer: int, reduce: int, inner: int) -> int:
+    """Remembered per argument tuple: the slicing decision depends on the arguments alone."""
+    return _lib.load().ak_reduce_workspace_bytes(dtype, outer, reduce, inner)
+
+
+def _reduce(name: str, y: torch.Tensor, x: torch.Tensor, outer: int, reduce: int, inner: int) -> None:
+    code = _code(x, name)
+    nbytes = _reduce_workspace_bytes(code, outer, reduce, inner) if inner > 1 else 0
+    if nbytes > 0:  # fp32 partial sums of row slices
+        ws = torch.empty(nbytes // 4, device=x.device, dtype=torch.float32)
+        _run(f"ak_{name}_ws", x, code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, ws.data_ptr(), nbytes,
+             shape=tuple(x.shape), dtype=x.dtype)
+        return
+    _run(f"ak_{name}", x, code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, shape=tuple(x.shape), dtype=x.dtype)
+
+
 def reduce_sum(y: torch.Tensor, x: torch.Tensor, outer: int, reduce: int, inner: int) -> None:
-    _run("ak_reduce_sum", x, _code(x, "reduce_sum"), x.data_ptr(), y.data_ptr(), outer, reduce, inner,
-         shape=tuple(x.shape), dtype=x.dtype)
+    _reduce("reduce_sum", y, x, outer, reduce, inner)
 
 
 def reduce_max(y: torch.Tensor, x: torch.Tensor, outer: int, reduce: int, inner: int) -> None:
-    _run("ak_reduce_max", x, _code(x, "reduce_max"), x.data_ptr(), y.data_ptr(), outer, reduce, inner,
-         shape=tuple(x.shape), dtype=x.dtype)
+    _reduce("reduce_max", y, x, outer, reduce, inner)
 
 
 def _ld(t: torch.Tensor) -> int:

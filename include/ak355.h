@@ -158,6 +158,21 @@ int ak_reduce_max(int dtype, const void* x, void* y, int64_t outer, int64_t redu
                   int64_t inner, hipStream_t stream);
 
 /*
+ * The same reductions with a caller-owned fp32 workspace, which lets a long reduction over a dim
+ * other than the last (inner > 1) run as row slices side by side, then add the slices in a fixed
+ * order (deterministic).
+ *   ak_reduce_workspace_bytes: bytes of workspace the shape uses; 0 when it would not slice.
+ *   With too small a workspace (or NULL) the call runs unsliced, as ak_reduce_sum / _max do.
+ * workspace: 4-byte aligned.
+ * Replaces: reference.py:72-78 reduce_sum_ref / reduce_max_ref over a dim other than the last.
+ */
+int64_t ak_reduce_workspace_bytes(int dtype, int64_t outer, int64_t reduce, int64_t inner);
+int ak_reduce_sum_ws(int dtype, const void* x, void* y, int64_t outer, int64_t reduce, int64_t inner,
+                     void* workspace, int64_t workspace_bytes, hipStream_t stream);
+int ak_reduce_max_ws(int dtype, const void* x, void* y, int64_t outer, int64_t reduce, int64_t inner,
+                     void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
+/*
  * GEMM with fp32 accumulation and one output rounding: C[M,N] = A[M,K] * op(B).
  *   b_trans = 0: B is [K, N] with row stride ldb  (torch.matmul(A, B), reference.py:10-12)
  *   b_trans = 1: B is [N, K] with row stride ldb  (x @ W.T for an nn.Linear weight W)

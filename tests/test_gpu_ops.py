@@ -607,6 +607,37 @@ def test_reduce_other_dims_and_max(gpu):
         assert torch.equal(reduce_mod.reduce_max(x.to(gpu), dim).cpu(), R.reduce_max_ref(x, dim))
 
 
+@pytest.mark.parametrize("shape,dim", [
+    ((8192, 512), 0), ((2, 192), 0), ((5000, 7), 0), ((3000, 1), 0), ((33, 1305), 0), ((4100, 100), 0),
+    ((3, 2100, 129), 1), ((40, 70, 33), 1), ((1, 9000, 8), 1), ((70000, 3, 2), 1),
+    ((513, 16, 64), 1), ((1025, 9), 0),
+])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+def test_reduce_strided_dim(gpu, shape, dim, dt):
+    """Reductions over a dim other than the last: column groups at the edges of a vector and a block,
+    row counts around a slice, sliced (workspace) and unsliced, with and without the workspace. An
+    fp32 sum of n terms in any order is within n 2^-24 sum|x| of the exact sum, plus one rounding."""
+    from autokernel_amd import _lib
+    x = torch.randn(*shape, generator=torch.Generator().manual_seed(3)).to(dt)
+    n, outer, inner = shape[dim], math.prod(shape[:dim]), math.prod(shape[dim + 1:])
+    xg = x.to(gpu)
+    y = kernels.get("reduce")(xg, dim)
+    exact = x.double().sum(dim)
+    u = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dt]
+    bound = n * 2.0 ** -24 * x.double().abs().sum(dim) + u * exact.abs() + 1e-30
+    assert y.dtype == dt and y.shape == exact.shape
+    assert bool(((y.double().cpu() - exact).abs() <= bound + (6e-8 if dt == torch.float16 else 0)).all())
+    y2 = torch.empty_like(y)  # no workspace: the unsliced form
+    _lib.check(_lib.load().ak_reduce_sum(_lib.DTYPE_CODE[dt], xg.data_ptr(), y2.data_ptr(), outer, n, inner,
+                                         _lib.stream_of(xg)), "ak_reduce_sum")
+    assert bool(((y2.double().cpu() - exact).abs() <= bound + (6e-8 if dt == torch.float16 else 0)).all())
+    xn = xg.clone()
+    xn[tuple(0 if d != dim else n // 2 for d in range(len(shape)))] = math.nan
+    assert torch.equal(reduce_mod.reduce_max(xg, dim), xg.max(dim).values)
+    m = reduce_mod.reduce_max(xn, dim)
+    assert torch.equal(torch.isnan(m), torch.isnan(xn.max(dim).values))
+
+
 def test_softmax_dim_and_layernorm_none(gpu):
     g = torch.Generator().manual_seed(8)
     x = torch.randn(33, 17, 5, generator=g)
