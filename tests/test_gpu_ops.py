@@ -319,6 +319,43 @@ def test_matmul_misaligned_operands_repacked(gpu, M, N, K, layout, dt):
     assert torch.equal(out, direct), f"repacked != element-load kernel {M}x{N}x{K} {layout} {dt}"
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (63, 65, 31), (64, 64, 32), (65, 3, 33), (129, 130, 64), (128, 127, 1000),
+                                   (2047, 2050, 100), (2048, 2048, 96), (300, 7, 15)])
+@pytest.mark.parametrize("bt", [True, False])
+def test_matmul_f32_tiles(gpu, M, N, K, bt):
+    """fp32 products at the edges of the 64 and 128 tiles and of the 32-deep k-tile, both layouts,
+    operands one element past a 16-byte boundary and row strides that are not vector multiples. Every
+    16 products are an fp32 chain (16 roundings of at most the chain's absolute sum) and the chains
+    add with compensation (2 roundings of the total): within 20 x 2^-24 of sum |a b|."""
+    g = torch.Generator().manual_seed(M * 3 + N + K)
+    A = torch.randn(M, K + 3, generator=g)
+    B = torch.randn(N, K + 5, generator=g) if bt else torch.randn(K, N + 5, generator=g)
+    Ad = A.to(gpu)[:, 1:K + 1]
+    Bd = B.to(gpu)[:, 1:K + 1].t() if bt else B.to(gpu)[:, 1:N + 1]
+    Ah, Bh = A[:, 1:K + 1].double(), (B[:, 1:K + 1].t() if bt else B[:, 1:N + 1]).double()
+    out = kernels.get("matmul")(Ad, Bd).double().cpu()
+    assert bool(((out - Ah @ Bh).abs() <= 20 * 2.0 ** -24 * (Ah.abs() @ Bh.abs())).all())
+
+
+@pytest.mark.parametrize("M,D,H", [(1, 1, 1), (65, 33, 31), (129, 100, 65), (2048, 64, 1100)])
+@pytest.mark.parametrize("act", ["silu", "relu2"])
+def test_gate_up_f32_tiles(gpu, M, D, H, act):
+    """fp32 gate/up at tile edges against 64 bits: each product within 20 x 2^-24 of its absolute sum,
+    carried through act(g) u (|act'| <= 1.1 for silu, 2 |g| for relu^2) plus four roundings."""
+    from autokernel_amd.kernels import _ops, host
+    g = torch.Generator().manual_seed(M + D + H)
+    x, wg, wu = torch.randn(M, D, generator=g), torch.randn(H, D, generator=g), torch.randn(H, D, generator=g)
+    h = torch.empty(M, H, device=gpu)
+    _ops.mlp_gate_up(h, x.to(gpu), wg.to(gpu), wu.to(gpu), host.ACTIVATIONS[act])
+    xd, gd, ud = x.double(), wg.double(), wu.double()
+    G, U = xd @ gd.T, xd @ ud.T
+    eg, eu = (20 * 2.0 ** -24 * (xd.abs() @ w.abs().T) for w in (gd, ud))
+    a = torch.nn.functional.silu(G) if act == "silu" else G.clamp(min=0) ** 2
+    slope = 1.1 if act == "silu" else 2 * (G.abs() + eg)
+    bound = slope * eg * (U.abs() + eu) + a.abs() * eu + 8 * 2.0 ** -24 * (a * U).abs() + 1e-30
+    assert bool(((h.double().cpu() - a * U).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 def test_matmul_batched_past_grid_z_limit(gpu, dt):
     """70000 items: past the 65535 a grid's z dimension holds, so ak_gemm_batched runs the batch in
