@@ -58,9 +58,12 @@ SIGNATURES: dict[str, list] = {
     "ak_set_launch_events": [_p, _p],
     "ak_flash_attn_fwd": [_i, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64,
                           _pi64, _pi64, _pi64, _pi64, _i, _f, _p],
+    "ak_flash_attn_workspace_bytes": [_i, _i64, _i64, _i64, _i64, _i64, _i64, _i],
+    "ak_flash_attn_fwd_ws": [_i, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64,
+                             _pi64, _pi64, _pi64, _pi64, _i, _f, _p, _i64, _p],
 }
 _STR_FUNCS = ("ak_version", "ak_status_string", "ak_last_hip_error_string")
-_I64_FUNCS = ("ak_gemm_workspace_bytes", "ak_reduce_workspace_bytes")  # return int64_t instead of a status
+_I64_FUNCS = ("ak_gemm_workspace_bytes", "ak_reduce_workspace_bytes", "ak_flash_attn_workspace_bytes")  # return int64_t instead of a status
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -24,7 +24,7 @@
 //     |score| enables an exact per-element emulation only when such a score exists.
 #include <limits.h>
 
-#include "ak_common.h"
+#include "attention_common.h"
 
 namespace ak {
 
@@ -37,7 +37,6 @@ constexpr float kFa2Slack = 8.0f;
 constexpr int kFaWaves = 4;                  // waves per block, 32 query rows each
 constexpr int kFaBQ = 32 * kFaWaves;         // query rows per block
 constexpr int kFaThreads = kFaWaves * 64;
-constexpr float kFaLog2e = 1.4426950408889634f;
 
 // 16-byte chunk c of an LDS row is stored at chunk c ^ (row & 7): a ds_read_b128 phase of 8 lanes
 // reading 8 consecutive rows at one logical chunk hits 8 different slots.
@@ -375,41 +374,9 @@ __device__ __forceinline__ u32x2 fa2_tr16(const uint16_t* p) {
       u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa2_s16x4*)(p)));
 }
 
-template <typename T>
-__device__ __forceinline__ uint32_t fa2_pack(float a, float b);
-template <>
-__device__ __forceinline__ uint32_t fa2_pack<TF16>(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, f16x2));
-}
-template <>
-__device__ __forceinline__ uint32_t fa2_pack<TBF16>(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, b2));
-}
-// acc + p.lo + p.hi (p: two packed values)
-template <typename T>
-__device__ __forceinline__ float fa2_sum2(uint32_t p, float acc);
-template <>
-__device__ __forceinline__ float fa2_sum2<TF16>(uint32_t p, float acc) {
-  const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
-  return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, p), one, acc, false);
-}
-template <>
-__device__ __forceinline__ float fa2_sum2<TBF16>(uint32_t p, float acc) {
-  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-  const b2 one = {(__bf16)1.0f, (__bf16)1.0f};
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, p), one, acc, false);
-}
 // Keeps the computation of x ahead of this point (an empty use the compiler cannot move).
 __device__ __forceinline__ void fa2_pin(const f32x16& x) { asm volatile("" ::"v"(x)); }
 // max over the two 32-lane halves (every lane gets the same value, combined in the same order)
-// NaN-propagating max (v_maximum3_f32 / v_maximum_f32). fmaxf would ignore a NaN score, and on
-// MFMA results the compiler then quiets each operand first (one v_max_f32 per operand: 11 more
-// instructions per 64-key tile). A row whose scores hold a NaN comes out NaN either way: its true
-// max fails the overflow test below.
-__device__ __forceinline__ float fa2_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 __device__ __forceinline__ float fa2_halves_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fa2_max(__uint_as_float(r[0]), __uint_as_float(r[1]));
@@ -1103,11 +1070,19 @@ static int launch_fa(const void* Q, const void* K, const void* V, void* O, int64
 
 using namespace ak;
 
-extern "C" int ak_flash_attn_fwd(int dtype, const void* Q, const void* K, const void* V, void* O,
-                                 int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk,
-                                 int64_t D, const int64_t* q_strides, const int64_t* k_strides,
-                                 const int64_t* v_strides, const int64_t* o_strides, int causal,
-                                 float sm_scale, hipStream_t stream) {
+extern "C" int64_t ak_flash_attn_workspace_bytes(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                                 int64_t Sk, int64_t D, int causal) {
+  if (dtype != AK_F16 && dtype != AK_BF16) return 0;
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Sq <= 0 || Sk <= 0 || D <= 0 || Hq % Hkv != 0) return 0;
+  if (B * Hq > INT_MAX || Sq > INT_MAX || Sk > INT_MAX) return 0;
+  return fa_rows_plan(B, Hq, Hkv, Sq, Sk, D, causal != 0).ws_bytes;
+}
+
+extern "C" int ak_flash_attn_fwd_ws(int dtype, const void* Q, const void* K, const void* V, void* O,
+                                    int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk,
+                                    int64_t D, const int64_t* q_strides, const int64_t* k_strides,
+                                    const int64_t* v_strides, const int64_t* o_strides, int causal,
+                                    float sm_scale, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   if (B < 0 || Hq < 0 || Hkv <= 0 || Sq < 0 || Sk < 0 || D <= 0) return AK_EINVAL;
   if (Hq % Hkv != 0) return AK_EINVAL;
   if (!q_strides || !k_strides || !v_strides || !o_strides) return AK_EINVAL;
@@ -1133,10 +1108,28 @@ extern "C" int ak_flash_attn_fwd(int dtype, const void* Q, const void* K, const 
       return launch_fa_general<TF16>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides, c, sm_scale, stream);
     return launch_fa_general<TBF16>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides, c, sm_scale, stream);
   }
+  // few query rows per KV head: keys split over waves and blocks
+  if (sm_scale > 0.f && fa_rows_plan(B, Hq, Hkv, Sq, Sk, D, c).ok) {
+    float* ws = host_aligned16(workspace) ? (float*)workspace : nullptr;
+    if (dtype == AK_F16)
+      return launch_fa_rows<TF16>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides,
+                                  sm_scale, ws, workspace_bytes, stream);
+    return launch_fa_rows<TBF16>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides,
+                                 sm_scale, ws, workspace_bytes, stream);
+  }
   if (dtype == AK_F16) {
     if (D == 64) return launch_fa<TF16, 64>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, q_strides, k_strides, v_strides, o_strides, c, sm_scale, stream);
     return launch_fa<TF16, 128>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, q_strides, k_strides, v_strides, o_strides, c, sm_scale, stream);
   }
   if (D == 64) return launch_fa<TBF16, 64>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, q_strides, k_strides, v_strides, o_strides, c, sm_scale, stream);
   return launch_fa<TBF16, 128>(Q, K, V, O, B, Hq, Hkv, Sq, Sk, q_strides, k_strides, v_strides, o_strides, c, sm_scale, stream);
+}
+
+extern "C" int ak_flash_attn_fwd(int dtype, const void* Q, const void* K, const void* V, void* O,
+                                 int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk,
+                                 int64_t D, const int64_t* q_strides, const int64_t* k_strides,
+                                 const int64_t* v_strides, const int64_t* o_strides, int causal,
+                                 float sm_scale, hipStream_t stream) {
+  return ak_flash_attn_fwd_ws(dtype, Q, K, V, O, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides, o_strides,
+                              causal, sm_scale, nullptr, 0, stream);
 }

@@ -1,20 +1,9 @@
-// gemm_common.h -- what the GEMM sources share: the MFMA wrapper, tile order, epilogue arguments and
+// gemm_common.h -- what the GEMM sources share: tile order, epilogue arguments and
 // the epilogue applied to a lane's accumulators (gemm.hip, gemm_f32.hip).
 #pragma once
-#include "ak_common.h"
+#include "mfma.h"
 
 namespace ak {
-
-template <typename T>
-__device__ __forceinline__ f32x4 mfma16x16x32(const u32x4& a, const u32x4& b, const f32x4& c);
-template <>
-__device__ __forceinline__ f32x4 mfma16x16x32<TF16>(const u32x4& a, const u32x4& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ f32x4 mfma16x16x32<TBF16>(const u32x4& a, const u32x4& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 // 4x8 transpose of 16-bit values: in[r] holds 8 n-values of k-row r; out[n] gets the 4 k-values
 // of column n (v_perm_b32 picks the low or high halves of two words).

@@ -300,10 +300,17 @@ void ak_op_flash_attn_fwd(at::Tensor& o, const at::Tensor& q, const at::Tensor& 
   const int64_t vs[3] = {v.stride(0), v.stride(1), v.stride(2)};
   const int64_t os[3] = {o.stride(0), o.stride(1), o.stride(2)};
   const c10::DeviceGuard g(q.device());
-  check_status(ak_flash_attn_fwd(dtype_code(q, op), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                 q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), q.size(3), qs, ks, vs, os,
-                                 causal ? 1 : 0, (float)sm_scale, stream_of(q)),
-               "ak_flash_attn_fwd");
+  const int code = dtype_code(q, op);
+  // fp32 partials of key slices (few query rows per KV head against many keys)
+  const int64_t bytes = ak_flash_attn_workspace_bytes(code, q.size(0), q.size(1), k.size(1), q.size(2), k.size(2),
+                                                      q.size(3), causal ? 1 : 0);
+  at::Tensor ws;
+  if (bytes > 0) ws = at::empty({bytes / 4}, q.options().dtype(at::kFloat));
+  check_status(ak_flash_attn_fwd_ws(code, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), q.size(0),
+                                    q.size(1), k.size(1), q.size(2), k.size(2), q.size(3), qs, ks, vs, os,
+                                    causal ? 1 : 0, (float)sm_scale, bytes > 0 ? ws.data_ptr() : nullptr, bytes,
+                                    stream_of(q)),
+               "ak_flash_attn_fwd_ws");
 }
 
 TORCH_LIBRARY_EXPAND(TORCH_EXTENSION_NAME, ops) {

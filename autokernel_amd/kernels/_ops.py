@@ -191,12 +191,26 @@ def mlp_gate_up(h: torch.Tensor, x: torch.Tensor, w_gate: torch.Tensor, w_up: to
          M, H, D, int(activation), M=M, H=H, D=D, dtype=x.dtype)
 
 
+@functools.lru_cache(maxsize=1024)
+def _attn_workspace_bytes(dtype: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int, causal: bool) -> int:
+    return _lib.load().ak_flash_attn_workspace_bytes(dtype, B, Hq, Hkv, Sq, Sk, D, int(causal))
+
+
 def flash_attn_fwd(o: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool,
                    sm_scale: float) -> None:
     """Q, O [B, Hq, Sq, D], K, V [B, Hkv, Sk, D], any strides with a contiguous head_dim."""
     B, Hq, Sq, D = q.shape
     Hkv, Sk = k.shape[1], k.shape[2]
     st = [_lib.i64_array(t.stride()[:3]) for t in (q, k, v, o)]
-    _run("ak_flash_attn_fwd", q, _code(q, "flash_attention"), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+    code = _code(q, "flash_attention")
+    # fp32 partials of key slices: only calls with few query rows per KV head have any
+    nbytes = _attn_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, bool(causal)) if Sq <= 16 else 0
+    if nbytes > 0:
+        ws = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
+        _run("ak_flash_attn_fwd_ws", q, code, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, Hq, Hkv, Sq,
+             Sk, D, st[0], st[1], st[2], st[3], int(bool(causal)), float(sm_scale), ws.data_ptr(), nbytes,
+             Q=tuple(q.shape), K=tuple(k.shape), dtype=q.dtype)
+        return
+    _run("ak_flash_attn_fwd", q, code, q.data_ptr(), k.data_ptr(), v.data_ptr(),
          o.data_ptr(), B, Hq, Hkv, Sq, Sk, D, st[0], st[1], st[2], st[3], int(bool(causal)), float(sm_scale),
          Q=tuple(q.shape), K=tuple(k.shape), dtype=q.dtype)

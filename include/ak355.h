@@ -313,6 +313,23 @@ int ak_flash_attn_fwd(int dtype, const void* Q, const void* K, const void* V, vo
                       const int64_t* v_strides, const int64_t* o_strides,
                       int causal, float sm_scale, hipStream_t stream);
 
+/*
+ * The same with a caller-owned workspace (16-byte aligned), which lets calls with few query rows per
+ * KV head and many keys (decode) split the keys over blocks: fp32 partial results, merged in a fixed
+ * order by a second launch (deterministic).
+ *   ak_flash_attn_workspace_bytes: bytes of workspace the shape uses; 0 when it would not split.
+ *   With too small a workspace (or NULL) the call runs unsplit, as ak_flash_attn_fwd does.
+ * Replaces: reference.py:32-42 flash_attention_ref for one or a few queries against cached keys.
+ */
+int64_t ak_flash_attn_workspace_bytes(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk,
+                                      int64_t D, int causal);
+int ak_flash_attn_fwd_ws(int dtype, const void* Q, const void* K, const void* V, void* O,
+                         int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D,
+                         const int64_t* q_strides, const int64_t* k_strides,
+                         const int64_t* v_strides, const int64_t* o_strides,
+                         int causal, float sm_scale, void* workspace, int64_t workspace_bytes,
+                         hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

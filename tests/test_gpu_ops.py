@@ -601,6 +601,45 @@ def test_attention_decode_shapes(gpu, D, dt, Sk, causal):
         assert torch.equal(out, V.repeat_interleave(4, 1)[:, :, :1]), "causal decode row is V[0]"
 
 
+@pytest.mark.parametrize("D,dt", [(64, torch.float16), (128, torch.float16), (64, torch.bfloat16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("B,Hq,Hk,Sq,Sk", [
+    (1, 1, 1, 1, 1), (1, 2, 2, 1, 31), (2, 8, 2, 1, 33), (1, 8, 1, 2, 127), (1, 4, 4, 16, 129), (1, 24, 1, 1, 300),
+    (3, 16, 1, 3, 1023), (1, 4, 1, 1, 1024), (1, 8, 2, 1, 1025), (2, 4, 2, 5, 4099), (1, 1, 1, 1, 20000),
+])
+def test_attention_few_rows(gpu, D, dt, B, Hq, Hk, Sq, Sk):
+    """Few query rows per KV head (attention_rows.hip): rows at the edges of a 16-row block, keys around
+    a step, a wave's and a slice's end, unsplit and split (with a workspace and, through the plain
+    entry point, without), K and V as views of longer caches whose other rows are NaN, f16 scores
+    past the overflow threshold. P is rounded to the element type (unit u) with an fp32 sum of the
+    rounded weights, then O once: within (2 u + Sk 2^-22) max|V| of the exact result."""
+    from autokernel_amd import _lib
+    g = torch.Generator().manual_seed(B + Hq + Sq + Sk + D)
+    Q = torch.randn(B, Hq, Sq, D, generator=g).to(dt)
+    cache = torch.full((2, B, Hk, Sk + 40, D), math.nan).to(dt)
+    cache[:, :, :, 8:8 + Sk] = torch.randn(2, B, Hk, Sk, D, generator=g).to(dt)
+    Qd, (K, V) = Q.to(gpu), (t[:, :, 8:8 + Sk] for t in cache.to(gpu))
+    rep = Hq // Hk
+    Kf, Vf = (t[:, :, 8:8 + Sk].double().repeat_interleave(rep, 1) for t in cache)
+    exact = (Q.double() @ Kf.transpose(2, 3) * D ** -0.5).softmax(-1) @ Vf
+    u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    bound = (2 * u + Sk * 2.0 ** -22) * Vf.abs().max()
+    out = kernels.get("flash_attention")(Qd, K, V, False)
+    assert float((out.double().cpu() - exact).abs().max()) <= bound
+    assert torch.equal(out, kernels.get("flash_attention")(Qd, K, V, False))
+    plain = torch.empty_like(out)
+    st = [_lib.i64_array(t.stride()[:3]) for t in (Qd, K, V, plain)]
+    _lib.check(_lib.load().ak_flash_attn_fwd(_lib.DTYPE_CODE[dt], Qd.data_ptr(), K.data_ptr(), V.data_ptr(),
+                                             plain.data_ptr(), B, Hq, Hk, Sq, Sk, D, *st, 0, D ** -0.5,
+                                             _lib.stream_of(Qd)), "ak_flash_attn_fwd")
+    assert float((plain.double().cpu() - exact).abs().max()) <= bound
+    if dt == torch.float16:  # the last key's score overflows f16 in every row of the first KV head
+        Qo, Ko = torch.full_like(Qd, 40.0), K.clone()
+        Ko[0, 0, Sk - 1] = 40.0
+        o = kernels.get("flash_attention")(Qo, Ko, V, False)
+        nan = torch.isnan(o)
+        assert bool(nan[0, :rep].all()) == (1600 * D >= 65520) and not bool(nan[0, rep:].any())
+
+
 def test_attention_rectangular_and_scale(gpu):
     g = torch.Generator().manual_seed(6)
     Q = torch.randn(1, 4, 96, 64, generator=g).bfloat16()
