@@ -663,6 +663,23 @@ static void launch_gemm_dma(const void* A, const void* B0, const void* B1, void*
   }
 }
 
+// Products of at most kSmallM rows on operands the LDS-DMA kernel can read: whether gemm_small is the
+// faster one. Measured (bf16, three rotating operand sets, us, LDS-DMA unsplit / gemm_small, M = 1, 16,
+// 32, 64; "nt" is an [N, K] B):
+//   nt N 2304 K 768    5.6 5.9 5.8 5.9 / 4.3 4.8 5.2 6.4     nt N 4096 K 4096   19.2 19.3 19.7 20.6 / 9.3 11.2 14.6 18.5
+//   nt N 4096 K 11008  56 58 60 75 / 18 26 35 45             nt N 8192 K 4096   20.0 20.0 20.5 21.5 / 19.4 21.7 26.0 26.3
+//   nn N 768 K 2048    10.0 10.1 10.2 10.4 / 5.4 6.1 6.2 6.5 nn N 4096 K 768    5.5 5.7 5.8 5.9 / 5.4 5.7 6.7 6.8
+//   nn N 4096 K 4096   18.9 19.1 19.2 20.6 / 15.3 16.0 18.8 18.7
+// Past N = 4096 the LDS-DMA kernel's tiles fill enough of the chip, and below K = 512 both are launches.
+// Gate/up (LDS-DMA / gemm_small, M = 1, 16, 32, 64): 4096 -> 11008 65 65 66 65 / 50 55 61 81, 768 -> 2048
+// 10.5 12.5 10.6 10.8 / 5.0 5.4 6.8 6.6, 192 -> 11648 7.3 7.3 7.5 8.1 / 7.7 8.1 6.9 9.7.
+static bool small_rows_win(int64_t M, int64_t N, int64_t K, bool bt, int nb) {
+  if (nb == 2) return N <= 4096 || (M <= 32 && K >= 512);
+  if (N > 4096 || K < 512) return false;
+  if (bt) return M <= 32 || N <= 1024 || K >= 2048;
+  return N <= 2560 || K >= 2048;
+}
+
 template <typename T, int NB, int EPI>
 static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C, int64_t M,
                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, bool bt,
@@ -670,20 +687,24 @@ static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C,
   // vec: A and B load as 16-byte k-chunks (C's alignment does not matter: the epilogue checks each
   // 8-byte store)
   bool vec = K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && host_aligned16(A) && host_aligned16(B0) &&
-             (!B1 || EPI == kEpiBias || EPI == kEpiBiasGelu || host_aligned16(B1)) && ep.batch_a % 8 == 0 &&
-             ep.batch_b % 8 == 0;
+             (!B1 || EPI == kEpiBias || EPI == kEpiBiasGelu || host_aligned16(B1));
   if (!bt) vec = vec && N % 8 == 0;
   const int m = (int)M, n = (int)N, k = (int)K;
-  // LDS-DMA path: nn.Linear-layout B, K a multiple of 64, 32-bit element offsets
-  const bool fits32 = M * lda < INT_MAX && N * ldb < INT_MAX;
-  if (bt && vec && K % kBK == 0 && K > 0 && fits32) {
+  // LDS-DMA path: K a multiple of 64, 32-bit element offsets
+  const bool dma = vec && K % kBK == 0 && K > 0 && (bt || N >= 8) && M * lda < INT_MAX &&
+                   (bt ? N : K) * ldb < INT_MAX;
+  // Few rows: always for operands that path cannot read, by shape for those it can. The batch (its
+  // strides included) has no say, so that every item of a batched product equals the 2-D product.
+  if (M <= kSmallM && K > 0 && (bt || NB == 1) && (!dma || small_rows_win(M, N, K, bt, NB)))
+    return launch_gemm_small<T, NB, EPI>(A, B0, B1, C, M, N, K, lda, ldb, ldc, bt, s, ep);
+  vec = vec && ep.batch_a % 8 == 0 && ep.batch_b % 8 == 0;
+  if (bt && dma && vec) {
     launch_gemm_dma<T, NB, EPI, false>(A, B0, B1, C, m, n, k, lda, ldb, ldc, s, ep);
     return record_launch();
   }
   // [K, N] B (torch.matmul's layout) on the same pipeline, fragments read through LDS transposes
   if constexpr (NB == 1) {
-    const bool fits32_kn = M * lda < INT_MAX && K * ldb < INT_MAX;
-    if (!bt && vec && K % kBK == 0 && K > 0 && N >= 8 && fits32_kn) {
+    if (!bt && dma && vec) {
       launch_gemm_dma<T, 1, EPI, true>(A, B0, B1, C, m, n, k, lda, ldb, ldc, s, ep);
       return record_launch();
     }
@@ -734,6 +755,17 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ w
 // 64-deep tiles) and a multiple of 64, and slices stop doubling once tiles x slices would pass the
 // CU count.
 static int splitk_slices(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, bool bt) {
+  if (M <= kSmallM) {
+    // gemm_small splits K inside its blocks, and is the faster one while its few columns are read by
+    // 16 rows or fewer or the matrix is small (us, split LDS-DMA / gemm_small: nt 16 x 4096 x 4096 14.2 /
+    // 11.2, nt 64 x 768 x 11008 26.8 / 22.9, nn 16 x 4096 x 2048 12.9 / 9.8; but nt 32 x 4096 x 11008
+    // 31.8 / 35.3, nn 16 x 4096 x 4096 14.4 / 16.0)
+    if (bt ? N <= 1024 || (N <= 4096 && M <= 16) : (N <= 768 && K <= 8192) || (N <= 4096 && K < 4096)) return 1;
+    // more than 128 tiles of 64 columns fill the chip unsplit (nt 16 x 11008 x 4096: 18.2 us against 21.6
+    // in two slices of 128 x 128 tiles; 128 tiles, N = 8192: 20.0 against 16.1); a deep [K, N] B still
+    // gains (nn 32 x 11008 x 11008: 55.1 us split, 59.4 unsplit)
+    if (cdiv(N, 64) > 128 && (bt || K <= 8192)) return 1;
+  }
   if (M <= 0 || N <= 0 || K <= 0 || N % 4 != 0 || ldc % 4 != 0 || lda % 8 != 0 || ldb % 8 != 0) return 1;
   if (M * lda >= INT_MAX || (bt ? N : K) * ldb >= INT_MAX || M * N * 8 >= INT_MAX) return 1;
   // [K, N] B runs the LDS-DMA kernel only with N a multiple of 8 (its 16-byte column chunks), the

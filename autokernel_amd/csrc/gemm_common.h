@@ -294,6 +294,12 @@ __device__ __forceinline__ void tile_epilogue(uint16_t* __restrict__ C, const ui
   }
 }
 
+// Products with at most kSmallM rows of A (gemm_small.hip); any alignment, any K > 0.
+constexpr int64_t kSmallM = 64;
+template <typename T, int NB, int EPI>
+int launch_gemm_small(const void* A, const void* B0, const void* B1, void* C, int64_t M, int64_t N, int64_t K,
+                      int64_t lda, int64_t ldb, int64_t ldc, bool bt, hipStream_t s, const EpiArgs& ep);
+
 // fp32 products (gemm_f32.hip). batch > 1: grid z is the batch item, whose operands start z * batch_x
 // elements further.
 int launch_gemm32(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,

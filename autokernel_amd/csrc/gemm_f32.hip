@@ -283,6 +283,16 @@ static bool small_tile32(int64_t M, int64_t N, int64_t batch, int bn_big) {
   return 1.15 * (double)small < (double)big;
 }
 
+// Few rows (gemm_small) instead of tiles: not for wide, shallow or very wide products of more than 32
+// (16) rows, whose tiles fill the chip (us, tiles / gemm_small: 48 x 50257 x 768 84 / 108, 33 x 14976 x 179
+// 10.8 / 15.1, gate/up 64 x 5120 -> 13824 264 / 317; but 64 x 11008 x 4096 142 / 123, 64 x 4096 x 4096
+// 142 / 38).
+static bool small_rows32(int64_t M, int64_t N, int64_t K) {
+  if (M > kSmallM || K == 0) return false;
+  if (M > 32 && N > 4096 && (N > 12288 || K < 1024)) return false;
+  return !(M > 16 && N > 8192 && K < 512);
+}
+
 template <int BM, int BN, int WM, int WN, int NB, bool BT>
 static void launch_tile32(const void* A, const void* B0, const void* B1, void* C, int64_t M, int64_t N, int64_t K,
                           int64_t lda, int64_t ldb, int64_t ldc, int act, hipStream_t s, int batch, int64_t ba,
@@ -296,6 +306,14 @@ static void launch_tile32(const void* A, const void* B0, const void* B1, void* C
 int launch_gemm32(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                   int64_t ldb, int64_t ldc, bool bt, hipStream_t s, int batch, int64_t batch_a, int64_t batch_b,
                   int64_t batch_c) {
+  if (small_rows32(M, N, K)) {
+    EpiArgs ep;
+    ep.batch = batch;
+    ep.batch_a = batch_a;
+    ep.batch_b = batch_b;
+    ep.batch_c = batch_c;
+    return launch_gemm_small<TF32, 1, kEpiStore>(A, B, nullptr, C, M, N, K, lda, ldb, ldc, bt, s, ep);
+  }
 #define AK_T32(BM, WN, BT) \
   launch_tile32<BM, BM, 2, WN, 1, BT>(A, B, nullptr, C, M, N, K, lda, ldb, ldc, 0, s, batch, batch_a, batch_b, batch_c)
   if (small_tile32(M, N, batch, 128)) {
@@ -311,6 +329,15 @@ int launch_gemm32(const void* A, const void* B, void* C, int64_t M, int64_t N, i
 
 int launch_gate_up32(const void* x, const void* wg, const void* wu, void* h, int64_t M, int64_t H, int64_t D,
                      int epi, hipStream_t s) {
+  if (small_rows32(M, H, D)) {
+    const EpiArgs ep;
+    switch (epi) {
+      case kEpiSilu: return launch_gemm_small<TF32, 2, kEpiSilu>(x, wg, wu, h, M, H, D, D, D, H, true, s, ep);
+      case kEpiGelu: return launch_gemm_small<TF32, 2, kEpiGelu>(x, wg, wu, h, M, H, D, D, D, H, true, s, ep);
+      case kEpiRelu2: return launch_gemm_small<TF32, 2, kEpiRelu2>(x, wg, wu, h, M, H, D, D, D, H, true, s, ep);
+      default: return launch_gemm_small<TF32, 2, kEpiNone>(x, wg, wu, h, M, H, D, D, D, H, true, s, ep);
+    }
+  }
   if (small_tile32(M, H, 1, 64))
     launch_tile32<64, 32, 2, 2, 2, true>(x, wg, wu, h, M, H, D, D, D, H, epi, s, 1, 0, 0, 0);
   else

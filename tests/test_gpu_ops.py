@@ -319,6 +319,61 @@ def test_matmul_misaligned_operands_repacked(gpu, M, N, K, layout, dt):
     assert torch.equal(out, direct), f"repacked != element-load kernel {M}x{N}x{K} {layout} {dt}"
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (1, 31, 8), (16, 33, 31), (17, 64, 33), (33, 65, 100), (64, 1000, 1029), (5, 4095, 2048), (32, 4097, 516),
+    (48, 4100, 40), (16, 8195, 70), (64, 3000, 2112), (7, 700, 4100), (1, 4096, 512), (64, 130, 9000),
+])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+def test_matmul_few_rows(gpu, M, N, K, dt):
+    """At most 64 rows (gemm_small.hip): both B layouts, aligned and with every operand one element past
+    a vector boundary in rows padded by an odd count (the padding is NaN), N and K at the edges of the
+    16-, 32- and 64-column blocks, of a k-step and of the waves' groups. fp32 accumulation: K 2^-24
+    sum|a b|, fp32 products additionally chained in 16s with compensation (20 x 2^-24), then one rounding.
+    Batched items equal the 2-D product bit for bit."""
+    g = torch.Generator().manual_seed(M + 3 * N + K)
+    u = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dt]
+
+    def odd(t):  # the same values as a view at an odd offset of NaN-padded rows
+        p = torch.full((t.shape[0], t.shape[1] + 3), math.nan, dtype=dt, device=gpu)
+        p[:, 1:1 + t.shape[1]] = t
+        return p[:, 1:1 + t.shape[1]]
+    A = (torch.randn(M, K, generator=g) / K ** 0.5).to(dt)
+    B = torch.randn(K, N, generator=g).to(dt)
+    exact, scale = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    bound = (20 if dt == torch.float32 else K) * 2.0 ** -24 * scale + u * exact.abs() + (6e-8 if dt == torch.float16 else 1e-38)
+    Ad, Bn, Bt = A.to(gpu), B.to(gpu), B.t().contiguous().to(gpu)
+    for name, a, b in (("kn", Ad, Bn), ("nk", Ad, Bt.t()), ("kn odd", odd(Ad), odd(Bn)), ("nk odd", odd(Ad), odd(Bt).t())):
+        out = kernels.get("matmul")(a, b)
+        assert bool(((out.double().cpu() - exact).abs() <= bound).all()), (name, M, N, K)
+    from autokernel_amd.kernels.host import _gemm
+    batch = torch.stack([Ad, Ad])
+    assert torch.equal(kernels.get("matmul")(batch, torch.stack([Bn, Bn]))[1], _gemm(Ad, Bn))
+    assert torch.equal(kernels.get("matmul")(batch, torch.stack([Bt, Bt]).transpose(1, 2))[1], _gemm(Ad, Bt.t()))
+
+
+@pytest.mark.parametrize("M,D,H", [(1, 513, 77), (16, 512, 4097), (17, 600, 5000), (33, 1000, 4096), (64, 31, 33), (64, 700, 5000)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("act", ["silu", "gelu", "relu2", "none"])
+def test_gate_up_few_rows(gpu, M, D, H, dt, act):
+    """Gate/up with at most 64 rows against the same products from matmul's path and the activation in
+    torch, each step rounded as the op rounds it: within two roundings of each factor where the two
+    sums round differently."""
+    from autokernel_amd.kernels import _ops, host
+    g = torch.Generator().manual_seed(M + D + H)
+    x, wg, wu = (torch.randn(*s, generator=g).to(dt) for s in ((M, D), (H, D), (H, D)))
+    x = (x.float() / D ** 0.5).to(dt)
+    h = torch.empty(M, H, device=gpu, dtype=dt)
+    _ops.mlp_gate_up(h, x.to(gpu), wg.to(gpu), wu.to(gpu), host.ACTIVATIONS.get(act, host.ACT_NONE))
+    G, U = ((x.double() @ w.double().T).to(dt).double() for w in (wg, wu))
+    a = {"silu": torch.nn.functional.silu, "gelu": torch.nn.functional.gelu, "relu2": lambda t: t.clamp(min=0) ** 2,
+         "none": lambda t: t}[act](G).to(dt).double()
+    u = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 20 * 2.0 ** -24}[dt]
+    slope = (2 * G.abs() + 1 if act == "relu2" else 1.2)
+    eg, eu = ((2 * u * t.abs() + D * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)) for t, w in ((G, wg), (U, wu)))
+    bound = (slope * eg + 2 * u * a.abs()) * (U.abs() + eu) + a.abs() * eu + 2 * u * (a * U).abs() + (2e-7 if dt == torch.float16 else 1e-30)
+    assert bool(((h.double().cpu() - a * U).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (63, 65, 31), (64, 64, 32), (65, 3, 33), (129, 130, 64), (128, 127, 1000),
                                    (2047, 2050, 100), (2048, 2048, 96), (300, 7, 15)])
 @pytest.mark.parametrize("bt", [True, False])
