@@ -1,13 +1,23 @@
 // row_common.h -- the row-parallel scheme shared by rmsnorm, layernorm, softmax, cross_entropy
 // and the last-dim reductions.
 //
-// A row of `cols` elements is owned by a group of L lanes (L = 8 .. 1024). When the row start is
-// 16-byte aligned and cols is a multiple of the 16-byte vector width, each lane loads up to VPT
+// A row of `cols` elements is owned by a group of L lanes (L = 8 .. 1024). Each lane loads up to VPT
 // 16-byte vectors (vector v = lane_in_group + j * L) into fp32 registers, so the row is read from
 // HBM exactly once and written once. Groups narrower than a wave share the wave (several rows per
 // wave, segmented butterflies); groups wider than a wave combine their per-wave partials through
-// LDS in a fixed order. Rows that are misaligned or too wide for registers use the looped kernels
+// LDS in a fixed order. Rows narrower than a vector or too wide for registers use the looped kernels
 // (one 256-thread block per row, scalar loads, two passes).
+//
+// ANY: rows of any width >= one vector, at any alignment. 16-byte accesses take any alignment here, but
+// those that straddle a 16-byte boundary run at a fraction of the rate (cross-entropy f16 [4096, 16385]:
+// 43 us with every load straddling, 36 us so), so a row's vectors are the aligned 16-byte pieces of
+// memory it covers, except the first and the last, which are moved to start and end with the row.
+// The elements that such an end shares with its neighbour are left out of sums at the end (maxima
+// take them twice, and both lanes store the same values). Measured, f16, us, against the kernels such
+// rows took before (2-byte loads in two or three passes, dword pairs, fp32-cached blocks): layernorm
+// [4097, 4097] 46.0 -> 16.8, rmsnorm 27 -> 15, row sums 15.4 -> 8.5; softmax [4096, 50257] 185 -> 157,
+// [4096, 20001] 92 -> 62, [16000, 1235] 37 -> 15; cross-entropy fp32 [4096, 20001] 144 -> 58. Widths just
+// under 65536, whose rows take straddling vectors, are level (softmax [1024, 65535] 62 -> 66).
 #pragma once
 #include "ak_common.h"
 
@@ -66,38 +76,85 @@ struct RowGeom {
   __device__ __forceinline__ static int group() { return threadIdx.x / L; }
 };
 
-// A row cached in fp32 registers: f[j * kVec + e] is element (lane + j * L) * kVec + e.
-template <typename T, int L, int VPT>
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <bool ANY>
+__device__ __forceinline__ u32x4 ldv(const void* p) {
+  if constexpr (ANY) return *reinterpret_cast<const u32x4_any*>(p);
+  else return ld16(p);
+}
+template <bool ANY>
+__device__ __forceinline__ void stv(void* p, const u32x4& v) {
+  if constexpr (ANY) *reinterpret_cast<u32x4_any*>(p) = v;
+  else st16(p, v);
+}
+
+// The vectors of a row: vector idx holds elements off(idx) .. off(idx) + kVec - 1 and counts those
+// in [lo, hi) of them.
+template <typename T, bool ANY>
+struct RowShape {
+  int cols, nvec, skew;  // skew: elements between the aligned address at or before the row and its start
+  // most: vectors the row's lanes hold. A row that an end piece would take past it (a width just under
+  // the widest one) takes its vectors from its own start instead.
+  __device__ __forceinline__ RowShape(const typename T::S* row, int cols_, bool active, int most = 1 << 30)
+      : cols(cols_) {
+    skew = ANY ? (int)(((uintptr_t)row & 15u) / sizeof(typename T::S)) : 0;
+    if (ANY && (cols + skew + T::kVec - 1) / T::kVec > most) skew = 0;
+    nvec = !active ? 0 : ANY ? (cols + skew + T::kVec - 1) / T::kVec : cols / T::kVec;
+  }
+  __device__ __forceinline__ int off(int idx) const {
+    return ANY ? min(max(idx * T::kVec - skew, 0), cols - T::kVec) : idx * T::kVec;
+  }
+  // fn(element) for the elements of vector idx that count; v holds the vector
+  template <typename F>
+  __device__ __forceinline__ void each(int idx, const float* v, F fn) const {
+    const int first = idx * T::kVec - skew;
+    if (!ANY || (first >= 0 && first + T::kVec <= cols)) {
+#pragma unroll
+      for (int e = 0; e < T::kVec; ++e) fn(v[e]);
+    } else {
+      const int lo = first < 0 ? 0 : first - (cols - T::kVec), hi = first < 0 ? T::kVec - skew : T::kVec;
+#pragma unroll
+      for (int e = 0; e < T::kVec; ++e)
+        if (e >= lo && e < hi) fn(v[e]);
+    }
+  }
+};
+
+// A row cached in fp32 registers: f[j * kVec + e] is element e of vector lane + j * L (0 past the row).
+template <typename T, int L, int VPT, bool ANY = false>
 struct RowRegs {
   static constexpr int kE = VPT * T::kVec;
   float f[kE];
 
   __device__ __forceinline__ static bool valid(int j, int gl, int nvec) { return gl + j * L < nvec; }
+  // fn(element) for every element of vector j that counts (the vector must be valid)
+  template <typename F>
+  __device__ __forceinline__ void each(int j, int gl, const RowShape<T, ANY>& sh, F fn) const {
+    sh.each(gl + j * L, f + j * T::kVec, fn);
+  }
 
-  __device__ __forceinline__ void load(const typename T::S* row, int nvec, int gl) {
+  __device__ __forceinline__ void load(const typename T::S* row, const RowShape<T, ANY>& sh, int gl) {
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const int idx = gl + j * L;
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (idx < nvec) v = ld16(row + (int64_t)idx * T::kVec);
+      if (idx < sh.nvec) v = ldv<ANY>(row + sh.off(idx));
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e) f[j * T::kVec + e] = T::lane_elem(v, e);
     }
   }
-  // Load a per-column vector (weights) with the same lane mapping.
-  __device__ __forceinline__ void load_cols(const typename T::S* w, int nvec, int gl) { load(w, nvec, gl); }
 
   // nt: nontemporal stores (outputs far larger than what a consumer could find in cache)
-  __device__ __forceinline__ void store(typename T::S* row, int nvec, int gl, bool nt = false) const {
+  __device__ __forceinline__ void store(typename T::S* row, const RowShape<T, ANY>& sh, int gl, bool nt = false) const {
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const int idx = gl + j * L;
-      if (idx < nvec) {
+      if (idx < sh.nvec) {
         u32x4 v;
 #pragma unroll
         for (int e = 0; e < T::kVec; ++e) T::set_elem(v, e, f[j * T::kVec + e]);
-        if (nt) st16_stream(row + (int64_t)idx * T::kVec, v);
-        else st16(row + (int64_t)idx * T::kVec, v);
+        if (nt) st16_stream(row + sh.off(idx), v);
+        else stv<ANY>(row + sh.off(idx), v);
       }
     }
   }
@@ -134,7 +191,25 @@ inline bool plan_row(int64_t nvec, int kvec, RowPlan* p, int want = 4) {
   return true;
 }
 
+// The plan for a row of `cols` elements; any: at any alignment (the most vectors it may cover, or, where
+// those do not fit, as many as it needs).
+inline bool plan_row_cols(int64_t cols, int kvec, bool any, RowPlan* p, int want = 4) {
+  if (cols < kvec) return false;
+  if (!any) return plan_row(cols / kvec, kvec, p, want);
+  return plan_row(cdiv(cols + kvec - 1, kvec), kvec, p, want) || plan_row(cdiv(cols, kvec), kvec, p, want);
+}
+
 }  // namespace ak
+
+// Expand a row-cached kernel launch over aligned rows (ANY false) and rows of any width (ANY true).
+#define AK_ANY_SWITCH(any, ...)       \
+  if (any) {                          \
+    constexpr bool ANY = true;        \
+    __VA_ARGS__;                      \
+  } else {                            \
+    constexpr bool ANY = false;       \
+    __VA_ARGS__;                      \
+  }
 
 // Expand a row-cached kernel launch over the supported (L, VPT) pairs.
 //   AK_ROW_SWITCH(plan, L, VPT, { launch<T, L, VPT>(...); })

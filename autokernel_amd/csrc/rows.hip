@@ -42,7 +42,7 @@ struct RmsStats {
   }
 };
 
-template <typename T, int L, int VPT, int FORM>
+template <typename T, int L, int VPT, int FORM, bool ANY>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void rmsnorm_rows(
     const typename T::S* __restrict__ x, const typename T::S* __restrict__ w,
     typename T::S* __restrict__ y, int64_t rows, int cols, float eps) {
@@ -51,26 +51,29 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void rmsnorm_rows(
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const int nvec = active ? cols / T::kVec : 0;
-  RowRegs<T, L, VPT> r;
-  r.load(x + row * cols, nvec, gl);
+  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
+  RowRegs<T, L, VPT, ANY> r;
+  r.load(x + row * cols, sh, gl);
   float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < RowRegs<T, L, VPT>::kE; ++e) ss += T::rnd(r.f[e] * r.f[e]);
+  for (int j = 0; j < VPT; ++j) {
+    if (!ANY || r.valid(j, gl, sh.nvec)) r.each(j, gl, sh, [&](float v) { ss += T::rnd(v * v); });
+  }
   ss = group_reduce<L, 0>(ss, red);
   const float inv = RmsStats<T, FORM>::scale(ss, cols, eps);
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int idx = gl + j * L;
-    if (idx < nvec) {
+    if (idx < sh.nvec) {
       // weights load here, after the reduction (measured faster than issuing them with the row:
       // 14.8 against 15.8 us for f16 4096x4096)
-      const u32x4 wv = ld16(w + (int64_t)idx * T::kVec);
+      const int off = sh.off(idx);
+      const u32x4 wv = ldv<ANY>(w + off);
       u32x4 o;
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e)
         T::set_elem(o, e, T::rnd(r.f[j * T::kVec + e] * inv) * T::lane_elem(wv, e));
-      st16(y + row * cols + (int64_t)idx * T::kVec, o);
+      stv<ANY>(y + row * cols + off, o);
     }
   }
 }
@@ -101,13 +104,13 @@ static int launch_rmsnorm(const void* x, const void* w, void* y, int64_t rows, i
   const S* wp = (const S*)w;
   S* yp = (S*)y;
   RowPlan plan;
-  const bool vec = cols % T::kVec == 0 && host_aligned16(x) && host_aligned16(y) && host_aligned16(w);
+  const bool any = cols % T::kVec != 0 || !host_aligned16(x) || !host_aligned16(y) || !host_aligned16(w);
   bool handled = false;
-  if (vec && plan_row(cols / T::kVec, T::kVec, &plan)) {
-    AK_ROW_SWITCH({
+  if (plan_row_cols(cols, T::kVec, any, &plan)) {
+    AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-      rmsnorm_rows<T, L, VPT, FORM><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, wp, yp, rows, (int)cols, eps);
-    });
+      rmsnorm_rows<T, L, VPT, FORM, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, wp, yp, rows, (int)cols, eps);
+    }));
   }
   if (!handled) rmsnorm_loop<T, FORM><<<(unsigned)rows, kLoopThreads, 0, s>>>(xp, wp, yp, (int)cols, eps);
   return record_launch();
@@ -126,41 +129,48 @@ __device__ __forceinline__ float ln_out(float v, float mean, float rstd, const t
   return o;
 }
 
-template <typename T, int L, int VPT>
+template <typename T, int L, int VPT, bool ANY>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void layernorm_rows(
     const typename T::S* __restrict__ x, const typename T::S* __restrict__ w,
     const typename T::S* __restrict__ b, typename T::S* __restrict__ y, int64_t rows, int cols,
     float eps) {
   using G = RowGeom<L>;
-  using R = RowRegs<T, L, VPT>;
+  using R = RowRegs<T, L, VPT, ANY>;
+  // With rows of any alignment the affine parameters load after the reductions, aligned ones with the
+  // row (us, after / with the row: f16 [4096, 16385] 74 / 99, aligned [4096, 4096] 15.5 / 13.7).
+  constexpr bool kAfter = ANY;
   __shared__ float red[G::kWPB];
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const int nvec = active ? cols / T::kVec : 0;
+  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
+  const int nvec = sh.nvec;
   R r;
-  r.load(x + row * cols, nvec, gl);
-  u32x4 wv[VPT], bv[VPT];  // affine parameters issued with the row, not after the reductions
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
+  r.load(x + row * cols, sh, gl);
+  u32x4 wv[VPT], bv[VPT];
+  auto affine = [&](int j) {
     const int idx = gl + j * L;
-    wv[j] = (w && idx < nvec) ? ld16(w + (int64_t)idx * T::kVec) : u32x4{0u, 0u, 0u, 0u};
-    bv[j] = (b && idx < nvec) ? ld16(b + (int64_t)idx * T::kVec) : u32x4{0u, 0u, 0u, 0u};
+    wv[j] = (w && idx < nvec) ? ldv<ANY>(w + sh.off(idx)) : u32x4{0u, 0u, 0u, 0u};
+    bv[j] = (b && idx < nvec) ? ldv<ANY>(b + sh.off(idx)) : u32x4{0u, 0u, 0u, 0u};
+  };
+  if constexpr (!kAfter) {
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) affine(j);
   }
   float s = 0.f;
 #pragma unroll
-  for (int e = 0; e < R::kE; ++e) s += r.f[e];  // invalid vectors hold 0
+  for (int j = 0; j < VPT; ++j) {
+    if (!ANY || R::valid(j, gl, nvec)) r.each(j, gl, sh, [&](float v) { s += v; });  // past the row: zeros
+  }
   const float mean = group_reduce<L, 0>(s, red) / (float)cols;
   float d = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
-    if (R::valid(j, gl, nvec)) {
-#pragma unroll
-      for (int e = 0; e < T::kVec; ++e) {
-        const float t = r.f[j * T::kVec + e] - mean;
+    if (R::valid(j, gl, nvec))
+      r.each(j, gl, sh, [&](float v) {
+        const float t = v - mean;
         d += t * t;
-      }
-    }
+      });
   }
   const float var = group_reduce<L, 0>(d, red) / (float)cols;
   const float rstd = rsqrtf(var + eps);
@@ -168,6 +178,7 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void layernorm_rows(
   for (int j = 0; j < VPT; ++j) {
     const int idx = gl + j * L;
     if (idx < nvec) {
+      if constexpr (kAfter) affine(j);
       u32x4 o;
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e) {
@@ -176,7 +187,7 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void layernorm_rows(
         if (b) v += T::lane_elem(bv[j], e);
         T::set_elem(o, e, v);
       }
-      st16(y + row * cols + (int64_t)idx * T::kVec, o);
+      stv<ANY>(y + row * cols + sh.off(idx), o);
     }
   }
 }
@@ -210,14 +221,14 @@ static int launch_layernorm(const void* x, const void* w, const void* b, void* y
   const S* bp = (const S*)b;
   S* yp = (S*)y;
   RowPlan plan;
-  const bool vec = cols % T::kVec == 0 && host_aligned16(x) && host_aligned16(y) &&
-                   (!w || host_aligned16(w)) && (!b || host_aligned16(b));
+  const bool any = cols % T::kVec != 0 || !host_aligned16(x) || !host_aligned16(y) ||
+                   (w && !host_aligned16(w)) || (b && !host_aligned16(b));
   bool handled = false;
-  if (vec && plan_row(cols / T::kVec, T::kVec, &plan)) {
-    AK_ROW_SWITCH({
+  if (plan_row_cols(cols, T::kVec, any, &plan)) {
+    AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-      layernorm_rows<T, L, VPT><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, wp, bp, yp, rows, (int)cols, eps);
-    });
+      layernorm_rows<T, L, VPT, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, wp, bp, yp, rows, (int)cols, eps);
+    }));
   }
   if (!handled) layernorm_loop<T><<<(unsigned)rows, kLoopThreads, 0, s>>>(xp, wp, bp, yp, (int)cols, eps);
   return record_launch();
@@ -226,22 +237,22 @@ static int launch_layernorm(const void* x, const void* w, const void* b, void* y
 // =============================================================================================
 // Softmax over the last dim (reference.py:15-17): fp32 max, exp and sum, one rounding.
 // =============================================================================================
-template <typename T, int L, int VPT>
+template <typename T, int L, int VPT, bool ANY>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
     const typename T::S* __restrict__ x, typename T::S* __restrict__ y, int64_t rows, int cols, int nt_out) {
   using G = RowGeom<L>;
-  using R = RowRegs<T, L, VPT>;
+  using R = RowRegs<T, L, VPT, ANY>;
   __shared__ float red[G::kWPB];
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const int nvec = active ? cols / T::kVec : 0;
+  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
   R r;
-  r.load(x + row * cols, nvec, gl);
+  r.load(x + row * cols, sh, gl);
   float m = -INFINITY;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
-    if (R::valid(j, gl, nvec))
+    if (R::valid(j, gl, sh.nvec))
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e) m = fmaxf(m, r.f[j * T::kVec + e]);
   m = group_reduce<L, 1>(m, red);
@@ -249,20 +260,17 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
-    if (R::valid(j, gl, nvec)) {
+    if (R::valid(j, gl, sh.nvec)) {
 #pragma unroll
-      for (int e = 0; e < T::kVec; ++e) {
-        const float p = fast_exp2(__builtin_fmaf(r.f[j * T::kVec + e], kLog2e, -mb));
-        r.f[j * T::kVec + e] = p;
-        s += p;
-      }
+      for (int e = 0; e < T::kVec; ++e) r.f[j * T::kVec + e] = fast_exp2(__builtin_fmaf(r.f[j * T::kVec + e], kLog2e, -mb));
+      r.each(j, gl, sh, [&](float p) { s += p; });
     }
   }
   s = group_reduce<L, 0>(s, red);
   const float inv = 1.0f / s;
 #pragma unroll
   for (int e = 0; e < R::kE; ++e) r.f[e] *= inv;
-  r.store(y + row * cols, nvec, gl, nt_out != 0);
+  r.store(y + row * cols, sh, gl, nt_out != 0);
 }
 
 // Online (max, sum-of-exp) accumulator used by the looped softmax and cross-entropy kernels.
@@ -290,193 +298,39 @@ __device__ __forceinline__ void block_combine_ms(OnlineMS a, float* red, float* 
   *S = tot;
 }
 
-// Wide rows that do not vectorise (a width that is not a multiple of the 16-byte vector, e.g. a
-// 50257-entry vocabulary): one row per block of 1024 threads, element c = tid + 1024 k cached in
-// registers (EPT per thread, so x is read once), with the vector path's arithmetic.
-// Rows are addressed through a buffer resource spanning the row (gfx9 descriptor word 3 =
-// 0x00020000, raw 32-bit data format, stride 0, num_records = the row's bytes): element c is one
-// per-thread VGPR offset plus a uniform scalar offset, where 64-bit pointers would take two VGPRs
-// per element and spill at this many elements per thread.
-constexpr int kWideThreads = 1024;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* row, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(row), (short)0, bytes, 0x00020000);
-}
-__device__ __forceinline__ void buf_ld(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint16_t& v) {
-  v = __builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0);
-}
-__device__ __forceinline__ void buf_ld(__amdgpu_buffer_rsrc_t r, int voff, int soff, float& v) {
-  v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-}
-__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint16_t v) {
-  __builtin_amdgcn_raw_buffer_store_b16(v, r, voff, soff, 0);
-}
-__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, int voff, int soff, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
-}
-
-// Loads this thread's EPT elements of the row (c = tid + 1024 k, c < cols) into v and returns
-// their maximum (-inf for a thread with none). Every load is issued before the first use so all
-// of them are in flight together, with no branch: a thread past the row's end re-reads element
-// cols - 1 (so every access stays in the row; a wave's such loads share one cache line) and takes
-// -inf by a select.
-template <typename T, int EPT>
-__device__ __forceinline__ float wide_load_max(const typename T::S* xr, int cols, float (&v)[EPT]) {
-  using S = typename T::S;
-  const __amdgpu_buffer_rsrc_t r = row_rsrc(xr, cols * (int)sizeof(S));
-  S e[EPT];
-#pragma unroll
-  for (int k = 0; k < EPT; ++k)
-    buf_ld(r, min((int)threadIdx.x + k * kWideThreads, cols - 1) * (int)sizeof(S), 0, e[k]);
-  float m = -INFINITY;
-#pragma unroll
-  for (int k = 0; k < EPT; ++k) {
-    v[k] = (int)threadIdx.x + k * kWideThreads < cols ? T::to_f(e[k]) : -INFINITY;
-    m = fmaxf(m, v[k]);
-  }
-  return m;
-}
-
-template <typename T, int EPT>
-__global__ __launch_bounds__(kWideThreads) void softmax_wide(const typename T::S* __restrict__ x,
-                                                             typename T::S* __restrict__ y, int cols) {
-  __shared__ float red[kWideThreads / kWave];
-  const int64_t base = (int64_t)blockIdx.x * cols;
-  float v[EPT];
-  float m = group_reduce<kWideThreads, 1>(wide_load_max<T, EPT>(x + base, cols, v), red);
-  const float mb = m * kLog2e;
-  // p is recomputed in the write pass rather than kept (the same expression, so the same value):
-  // holding both x and p would spill at 64 elements per thread.
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < EPT; ++k)
-    if (threadIdx.x + k * kWideThreads < cols) s += fast_exp2(__builtin_fmaf(v[k], kLog2e, -mb));
-  s = group_reduce<kWideThreads, 0>(s, red);
-  const float inv = 1.0f / s;
-  using S = typename T::S;
-  const __amdgpu_buffer_rsrc_t r = row_rsrc(y + base, cols * (int)sizeof(S));
-  const int voff = threadIdx.x * (int)sizeof(S);
-#pragma unroll
-  for (int k = 0; k < EPT; ++k)
-    if (threadIdx.x + k * kWideThreads < cols)
-      buf_st(r, voff, k * kWideThreads * (int)sizeof(S), T::from_f(fast_exp2(__builtin_fmaf(v[k], kLog2e, -mb)) * inv));
-}
-
-// Wide 16-bit rows of any width and alignment, held packed: one row per 1024-thread block with the
-// row's elements kept two per VGPR, as the 4-byte pairs memory already stores them. A block needs
-// about half the registers of softmax_wide, so two rows are in flight per CU (one block's
-// reductions and stores overlap the other's loads). Pair k of thread t is the aligned dword at
-// element par + 2 (t + 1024 k) of the row, par = 1 when the row's first element is the high half
-// of a dword (odd widths put every other row there). The element left at either end (the first
-// when par = 1, the last when cols - par is odd) is one extra value held by thread 0 (first) or 1
-// (last). Pairs past the row's end come back as zeros from the buffer's range check and are
-// masked by index. The whole byte offset of a load is its VGPR offset: on gfx9 the range check
-// covers the VGPR and instruction offsets, not the scalar offset, so a per-k scalar offset would let
-// reads run past the row (and, on a tensor's last row, past its allocation). Requires the output
-// rows to share the input rows' dword alignment.
-template <typename T, int NP>
-struct WidePairs {
-  uint32_t p[NP];
-  float xt;  // thread 0: the first element when par = 1; thread 1: the last when cols - par is odd
-  bool has_xt;
-  int npairs, par;
-
-  __device__ __forceinline__ static float lo(uint32_t w) { return T::to_f((uint16_t)(w & 0xffffu)); }
-  __device__ __forceinline__ static float hi(uint32_t w) { return T::to_f((uint16_t)(w >> 16)); }
-  __device__ __forceinline__ bool valid(int k) const { return (int)threadIdx.x + k * kWideThreads < npairs; }
-
-  // loads the row; returns this thread's maximum (-inf when it holds nothing)
-  __device__ __forceinline__ float load_max(const uint16_t* row, int cols) {
-    par = (int)(((uintptr_t)row >> 1) & 1u);
-    npairs = (cols - par) >> 1;
-    const __amdgpu_buffer_rsrc_t r = row_rsrc(row + par, npairs * 4);
-#pragma unroll
-    for (int k = 0; k < NP; ++k)
-      p[k] = __builtin_amdgcn_raw_buffer_load_b32(r, ((int)threadIdx.x + k * kWideThreads) * 4, 0, 0);
-    has_xt = (threadIdx.x == 0 && par) || (threadIdx.x == 1 && ((cols - par) & 1));
-    xt = has_xt ? T::to_f(row[threadIdx.x == 0 ? 0 : cols - 1]) : -INFINITY;
-    float m = xt;
-#pragma unroll
-    for (int k = 0; k < NP; ++k)
-      if (valid(k)) m = fmaxf(m, fmaxf(lo(p[k]), hi(p[k])));
-    return m;
-  }
-  // sum of f(x) over the thread's elements
-  template <typename F>
-  __device__ __forceinline__ float sum(F f) const {
-    float s = has_xt ? f(xt) : 0.f;
-#pragma unroll
-    for (int k = 0; k < NP; ++k)
-      if (valid(k)) s += f(lo(p[k])) + f(hi(p[k]));
-    return s;
-  }
-};
-
-template <typename T, int NP>
-__global__ __launch_bounds__(kWideThreads, 2) void softmax_wide_pairs(const uint16_t* __restrict__ x,
-                                                                     uint16_t* __restrict__ y, int cols) {
-  __shared__ float red[kWideThreads / kWave];
-  const int64_t base = (int64_t)blockIdx.x * cols;
-  WidePairs<T, NP> w;
-  const float m = group_reduce<kWideThreads, 1>(w.load_max(x + base, cols), red);
-  const float mb = m * kLog2e;
-  auto e = [&](float v) { return fast_exp2(__builtin_fmaf(v, kLog2e, -mb)); };
-  const float s = group_reduce<kWideThreads, 0>(w.sum(e), red);
-  const float inv = 1.0f / s;
-  uint16_t* yr = y + base;
-  const __amdgpu_buffer_rsrc_t r = row_rsrc(yr + w.par, w.npairs * 4);
-#pragma unroll
-  for (int k = 0; k < NP; ++k)
-    if (w.valid(k)) {
-      const uint32_t o = (uint32_t)T::from_f(e(w.lo(w.p[k])) * inv) | ((uint32_t)T::from_f(e(w.hi(w.p[k])) * inv) << 16);
-      __builtin_amdgcn_raw_buffer_store_b32(o, r, (int)threadIdx.x * 4, k * kWideThreads * 4, 0);
-    }
-  if (w.has_xt) yr[threadIdx.x == 0 ? 0 : cols - 1] = T::from_f(e(w.xt) * inv);
-}
-
-// Streaming row statistics for 16-bit rows that do not vectorise (softmax_stream, ce_stream): one
-// row per 256-thread block, read once as aligned dword pairs (the WidePairs layout) with an online
-// (max, sum) per thread and 8 pairs in flight per thread. Nothing is cached in registers, so up to
-// eight rows are in flight per CU. Per chunk of 16 elements: the chunk max (NaN-propagating), one
-// rescale of the running sum, then exp2((x - max) log2 e) per element; the per-thread (max, sum)
-// pairs combine in a fixed order (block_combine_ms), as in the looped kernels.
-constexpr int kStreamUnroll = 8;
+// Streaming row statistics (softmax_stream, ce_stream): one row per 256-thread block, read once as the
+// aligned 16-byte vectors it covers (row_common.h, ANY) with an online (max, sum) per thread and
+// kStreamUnroll vectors in flight. Nothing is cached in registers, so up to eight rows are in flight
+// per CU. Per chunk: the chunk max (NaN-propagating), one rescale of the running sum, then
+// exp2((x - max) log2 e) per element; the per-thread (max, sum) pairs combine in a fixed order
+// (block_combine_ms), as in the looped kernels.
+constexpr int kStreamUnroll = 4;
 template <typename T>
-__device__ __forceinline__ void stream_ms(const uint16_t* xr, int cols, float* red, float* M, float* S) {
-  const int par = (int)(((uintptr_t)xr >> 1) & 1u);
-  const int npairs = (cols - par) >> 1;
-  const __amdgpu_buffer_rsrc_t r = row_rsrc(xr + par, npairs * 4);
+__device__ __forceinline__ void stream_ms(const typename T::S* xr, int cols, float* red, float* M, float* S) {
+  const RowShape<T, true> sh(xr, cols, true);
   float m = -INFINITY, s = 0.f;
-  // fold a chunk with maximum cm and values v[0..n) into (m, s)
-  auto fold = [&](float cm, auto&& each) {
-    const float mn = __builtin_elementwise_maximum(m, cm);
-    if (mn == -INFINITY) return;  // nothing but -inf so far
-    s = (m == -INFINITY) ? 0.f : s * fast_exp2((m - mn) * kLog2e);
-    each([&](float v) { s += fast_exp2((v - mn) * kLog2e); });
-    m = mn;
-  };
-  if ((threadIdx.x == 0 && par) || (threadIdx.x == 1 && ((cols - par) & 1))) {
-    const float v = T::to_f(xr[threadIdx.x == 0 ? 0 : cols - 1]);
-    fold(v, [&](auto&& f) { f(v); });
-  }
-  for (int b = 0; b < npairs; b += kLoopThreads * kStreamUnroll) {
-    uint32_t p[kStreamUnroll];
+  for (int b = threadIdx.x; b < sh.nvec; b += kLoopThreads * kStreamUnroll) {
+    u32x4 p[kStreamUnroll];
 #pragma unroll
-    for (int u = 0; u < kStreamUnroll; ++u)
-      p[u] = __builtin_amdgcn_raw_buffer_load_b32(r, ((int)threadIdx.x + b + u * kLoopThreads) * 4, 0, 0);
+    for (int u = 0; u < kStreamUnroll; ++u)  // past the row: its last vector, left out of the sum
+      p[u] = ldv<true>(xr + sh.off(min(b + u * kLoopThreads, sh.nvec - 1)));
     float cm = -INFINITY;
 #pragma unroll
     for (int u = 0; u < kStreamUnroll; ++u)
-      if (b + u * kLoopThreads + (int)threadIdx.x < npairs)
-        cm = __builtin_elementwise_maximum(cm, __builtin_elementwise_maximum(WidePairs<T, 1>::lo(p[u]), WidePairs<T, 1>::hi(p[u])));
-    fold(cm, [&](auto&& f) {
 #pragma unroll
-      for (int u = 0; u < kStreamUnroll; ++u)
-        if (b + u * kLoopThreads + (int)threadIdx.x < npairs) {
-          f(WidePairs<T, 1>::lo(p[u]));
-          f(WidePairs<T, 1>::hi(p[u]));
-        }
-    });
+      for (int e = 0; e < T::kVec; ++e) cm = __builtin_elementwise_maximum(cm, T::lane_elem(p[u], e));
+    const float mn = __builtin_elementwise_maximum(m, cm);
+    if (mn == -INFINITY) continue;  // nothing but -inf so far
+    s = (m == -INFINITY) ? 0.f : s * fast_exp2((m - mn) * kLog2e);
+#pragma unroll
+    for (int u = 0; u < kStreamUnroll; ++u)
+      if (b + u * kLoopThreads < sh.nvec) {
+        float v[T::kVec];
+#pragma unroll
+        for (int e = 0; e < T::kVec; ++e) v[e] = T::lane_elem(p[u], e);
+        sh.each(b + u * kLoopThreads, v, [&](float x) { s += fast_exp2((x - mn) * kLog2e); });
+      }
+    m = mn;
   }
   OnlineMS a;
   a.m = m;
@@ -485,37 +339,30 @@ __device__ __forceinline__ void stream_ms(const uint16_t* xr, int cols, float* r
   block_combine_ms(a, red, M, S);
 }
 
-// Streaming softmax for 16-bit rows: the online pass above, then a second read of the row (from
-// the caches when they still hold it) that writes exp2((x - M) log2 e) / S as dword pairs.
+// Streaming softmax: the online pass above, then a second read of the row (from the caches when they
+// still hold it) that writes exp2((x - M) log2 e) / S.
 template <typename T>
-__global__ __launch_bounds__(kLoopThreads) void softmax_stream(const uint16_t* __restrict__ x,
-                                                               uint16_t* __restrict__ y, int cols) {
+__global__ __launch_bounds__(kLoopThreads) void softmax_stream(const typename T::S* __restrict__ x,
+                                                               typename T::S* __restrict__ y, int cols) {
   __shared__ float red[kLoopThreads / kWave];
-  const int64_t base = (int64_t)blockIdx.x * cols;
-  const uint16_t* xr = x + base;
-  uint16_t* yr = y + base;
+  const typename T::S* xr = x + (int64_t)blockIdx.x * cols;
+  typename T::S* yr = y + (int64_t)blockIdx.x * cols;
   float M, S;
   stream_ms<T>(xr, cols, red, &M, &S);
   const float inv = 1.0f / S;
-  auto e = [&](float v) { return T::from_f(fast_exp2((v - M) * kLog2e) * inv); };
-  const int par = (int)(((uintptr_t)xr >> 1) & 1u);
-  const int npairs = (cols - par) >> 1;
-  const __amdgpu_buffer_rsrc_t r = row_rsrc(xr + par, npairs * 4);
-  const __amdgpu_buffer_rsrc_t w = row_rsrc(yr + par, npairs * 4);
-  if ((threadIdx.x == 0 && par) || (threadIdx.x == 1 && ((cols - par) & 1))) {
-    const int c = threadIdx.x == 0 ? 0 : cols - 1;
-    yr[c] = e(T::to_f(xr[c]));
-  }
-  for (int b = 0; b < npairs; b += kLoopThreads * kStreamUnroll) {
-    uint32_t p[kStreamUnroll];
+  const RowShape<T, true> sh(xr, cols, true);
+  for (int b = threadIdx.x; b < sh.nvec; b += kLoopThreads * kStreamUnroll) {
+    u32x4 p[kStreamUnroll];
 #pragma unroll
     for (int u = 0; u < kStreamUnroll; ++u)
-      p[u] = __builtin_amdgcn_raw_buffer_load_b32(r, ((int)threadIdx.x + b + u * kLoopThreads) * 4, 0, 0);
+      p[u] = ldv<true>(xr + sh.off(min(b + u * kLoopThreads, sh.nvec - 1)));
 #pragma unroll
     for (int u = 0; u < kStreamUnroll; ++u)
-      if (b + u * kLoopThreads + (int)threadIdx.x < npairs) {
-        const uint32_t o = (uint32_t)e(WidePairs<T, 1>::lo(p[u])) | ((uint32_t)e(WidePairs<T, 1>::hi(p[u])) << 16);
-        __builtin_amdgcn_raw_buffer_store_b32(o, w, (int)threadIdx.x * 4, (b + u * kLoopThreads) * 4, 0);
+      if (b + u * kLoopThreads < sh.nvec) {
+        u32x4 o;
+#pragma unroll
+        for (int e = 0; e < T::kVec; ++e) T::set_elem(o, e, fast_exp2((T::lane_elem(p[u], e) - M) * kLog2e) * inv);
+        stv<true>(yr + sh.off(b + u * kLoopThreads), o);
       }
   }
 }
@@ -544,7 +391,6 @@ static int launch_softmax(const void* x, void* y, int64_t rows, int64_t cols, hi
   const S* xp = (const S*)x;
   S* yp = (S*)y;
   RowPlan plan;
-  const bool vec = cols % T::kVec == 0 && host_aligned16(x) && host_aligned16(y);
   bool handled = false;
   // An output larger than the 256 MB Infinity Cache is stored nontemporally; smaller outputs keep
   // plain stores, so the consumer that usually reads them next finds them in cache. Measured, f16
@@ -554,32 +400,14 @@ static int launch_softmax(const void* x, void* y, int64_t rows, int64_t cols, hi
   // (the dirty lines' write-back then lands in the next kernel): 56.3 against 67.3 us per
   // RoPE(q), RoPE(k), softmax step.
   const int nt_out = rows * cols * (int64_t)sizeof(S) > ((int64_t)256 << 20);
-  if (vec && plan_row(cols / T::kVec, T::kVec, &plan)) {
-    AK_ROW_SWITCH({
+  const bool any = cols % T::kVec != 0 || !host_aligned16(x) || !host_aligned16(y);
+  if (plan_row_cols(cols, T::kVec, any, &plan)) {
+    AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-      launch_timed(softmax_rows<T, L, VPT>, grid, dim3(RowGeom<L>::kThreads), 0, s, xp, yp, rows, (int)cols, nt_out);
-    });
-  }
-  // 16-bit rows that do not vectorise, when x and y rows share their dword alignment: the streaming
-  // kernel up to 32768 columns and past 65536, the packed register-cached one in between (measured,
-  // f16, 4096 rows: 16385 columns 67.0 us streaming / 99.3 us packed; 24577: 101 / 115; 32769: 138 /
-  // 136; 40961: 182 / 152; 50257: 230 / 180 (the fp32-cached kernel: 234.9)).
-  if constexpr (sizeof(S) == 2) {
-    if (!handled && cols > 4096 && ((((uintptr_t)x ^ (uintptr_t)y) & 3u) == 0)) {
-      const uint16_t* xs = (const uint16_t*)x;
-      uint16_t* ys = (uint16_t*)y;
-      if (cols > 32768 && cols <= 64 * kWideThreads)
-        launch_timed(softmax_wide_pairs<T, 32>, dim3((unsigned)rows), dim3(kWideThreads), 0, s, xs, ys, (int)cols);
-      else
-        launch_timed(softmax_stream<T>, dim3((unsigned)rows), dim3(kLoopThreads), 0, s, xs, ys, (int)cols);
-      handled = true;
-    }
-  }
-  if (!handled && cols > 4096 && cols <= 16 * kWideThreads) {
-    launch_timed(softmax_wide<T, 16>, dim3((unsigned)rows), dim3(kWideThreads), 0, s, xp, yp, (int)cols);
-    handled = true;
-  } else if (!handled && cols > 16 * kWideThreads && cols <= 64 * kWideThreads) {
-    launch_timed(softmax_wide<T, 64>, dim3((unsigned)rows), dim3(kWideThreads), 0, s, xp, yp, (int)cols);
+      launch_timed(softmax_rows<T, L, VPT, ANY>, grid, dim3(RowGeom<L>::kThreads), 0, s, xp, yp, rows, (int)cols, nt_out);
+    }));
+  } else if (cols >= T::kVec) {
+    launch_timed(softmax_stream<T>, dim3((unsigned)rows), dim3(kLoopThreads), 0, s, xp, yp, (int)cols);
     handled = true;
   }
   if (!handled) launch_timed(softmax_loop<T>, dim3((unsigned)rows), dim3(kLoopThreads), 0, s, xp, yp, (int)cols);
@@ -614,23 +442,23 @@ __device__ __forceinline__ float ce_row_loss_b2(const typename T::S* xr, int64_t
   return -lp;
 }
 
-template <typename T, int L, int VPT>
+template <typename T, int L, int VPT, bool ANY>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void ce_rows(
     const typename T::S* __restrict__ x, const int64_t* __restrict__ tgt, float* __restrict__ loss,
     int64_t rows, int cols, int64_t ignore_index) {
   using G = RowGeom<L>;
-  using R = RowRegs<T, L, VPT>;
+  using R = RowRegs<T, L, VPT, ANY>;
   __shared__ float red[G::kWPB];
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const int nvec = active ? cols / T::kVec : 0;
+  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
   R r;
-  r.load(x + row * cols, nvec, gl);
+  r.load(x + row * cols, sh, gl);
   float m = -INFINITY;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
-    if (R::valid(j, gl, nvec))
+    if (R::valid(j, gl, sh.nvec))
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e) m = fmaxf(m, r.f[j * T::kVec + e]);
   m = group_reduce<L, 1>(m, red);
@@ -638,38 +466,19 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void ce_rows(
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
-    if (R::valid(j, gl, nvec))
-#pragma unroll
-      for (int e = 0; e < T::kVec; ++e) s += fast_exp2(__builtin_fmaf(r.f[j * T::kVec + e], kLog2e, -mb));
+    if (R::valid(j, gl, sh.nvec)) r.each(j, gl, sh, [&](float v) { s += fast_exp2(__builtin_fmaf(v, kLog2e, -mb)); });
   s = group_reduce<L, 0>(s, red);
   if (active && gl == 0) loss[row] = ce_row_loss_b2<T>(x + row * cols, tgt[row], cols, ignore_index, mb, s);
 }
 
-template <typename T, int EPT>
-__global__ __launch_bounds__(kWideThreads) void ce_wide(const typename T::S* __restrict__ x,
-                                                        const int64_t* __restrict__ tgt, float* __restrict__ loss,
-                                                        int cols, int64_t ignore_index) {
-  __shared__ float red[kWideThreads / kWave];
-  const typename T::S* xr = x + (int64_t)blockIdx.x * cols;
-  float v[EPT];
-  const float m = group_reduce<kWideThreads, 1>(wide_load_max<T, EPT>(xr, cols, v), red);
-  const float mb = m * kLog2e;
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < EPT; ++k)
-    if (threadIdx.x + k * kWideThreads < cols) s += fast_exp2(__builtin_fmaf(v[k], kLog2e, -mb));
-  s = group_reduce<kWideThreads, 0>(s, red);
-  if (threadIdx.x == 0) loss[blockIdx.x] = ce_row_loss_b2<T>(xr, tgt[blockIdx.x], cols, ignore_index, mb, s);
-}
-
-// Cross-entropy of a 16-bit row from the streaming statistics: loss = x_t - M - log S, as in ce_loop.
+// Cross-entropy of a row from the streaming statistics: loss = x_t - M - log S, as in ce_loop.
 template <typename T>
-__global__ __launch_bounds__(kLoopThreads) void ce_stream(const uint16_t* __restrict__ x,
+__global__ __launch_bounds__(kLoopThreads) void ce_stream(const typename T::S* __restrict__ x,
                                                           const int64_t* __restrict__ tgt,
                                                           float* __restrict__ loss, int cols,
                                                           int64_t ignore_index) {
   __shared__ float red[kLoopThreads / kWave];
-  const uint16_t* xr = x + (int64_t)blockIdx.x * cols;
+  const typename T::S* xr = x + (int64_t)blockIdx.x * cols;
   float M, S;
   stream_ms<T>(xr, cols, red, &M, &S);
   if (threadIdx.x == 0) loss[blockIdx.x] = ce_row_loss<T>(xr, tgt[blockIdx.x], cols, ignore_index, M, S);
@@ -728,29 +537,21 @@ static int launch_ce(const void* logits, const int64_t* tgt, float* loss, void* 
   using S = typename T::S;
   const S* xp = (const S*)logits;
   RowPlan plan;
-  const bool vec = vocab % T::kVec == 0 && host_aligned16(logits);
+  const bool any = vocab % T::kVec != 0 || !host_aligned16(logits);
   bool handled = rows == 0;  // no rows: only the mean kernel runs (0 / 0 = NaN, as torch gives)
-  if (!handled && vec && plan_row(vocab / T::kVec, T::kVec, &plan)) {
-    AK_ROW_SWITCH({
+  const bool planned = plan_row_cols(vocab, T::kVec, any, &plan);
+  // 16-bit rows past 32768 columns, and unaligned ones past 16384, stream once the rows fill the chip: a
+  // register-cached block of theirs leaves room for one row per CU (us, ce_rows / ce_stream, f16: 4096 x
+  // 50264 98 / 81, 4096 x 32769 78 / 56, 4096 x 16385 36 / 30; but 100 x 65536 9.0 / 12.4, aligned 4096 x
+  // 32000 49.0 / 54.7, fp32 4096 x 16385 50 / 53).
+  const bool stream = sizeof(S) == 2 && rows > 512 && (vocab > 32768 || (any && vocab > 16384));
+  if (!handled && planned && !stream) {
+    AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-      ce_rows<T, L, VPT><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, tgt, loss, rows, (int)vocab, ignore_index);
-    });
-  }
-  // 16-bit rows that do not vectorise: the streaming kernel at any width past 4096 (measured, f16:
-  // 8192 x 50257 152.5 us against 216.1 register-cached packed and 274.1 fp32-cached; 4096 x 16385
-  // 33.0 against 80.1). For rows that vectorise the register-cached ce_rows stays faster (4096 x
-  // 32000: 51.6 against 57.1 streaming).
-  if constexpr (sizeof(S) == 2) {
-    if (!handled && vocab > 4096) {
-      ce_stream<T><<<(unsigned)rows, kLoopThreads, 0, s>>>((const uint16_t*)logits, tgt, loss, (int)vocab, ignore_index);
-      handled = true;
-    }
-  }
-  if (!handled && vocab > 4096 && vocab <= 16 * kWideThreads) {
-    ce_wide<T, 16><<<(unsigned)rows, kWideThreads, 0, s>>>(xp, tgt, loss, (int)vocab, ignore_index);
-    handled = true;
-  } else if (!handled && vocab > 16 * kWideThreads && vocab <= 64 * kWideThreads) {
-    ce_wide<T, 64><<<(unsigned)rows, kWideThreads, 0, s>>>(xp, tgt, loss, (int)vocab, ignore_index);
+      ce_rows<T, L, VPT, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, tgt, loss, rows, (int)vocab, ignore_index);
+    }));
+  } else if (!handled && vocab >= T::kVec) {
+    ce_stream<T><<<(unsigned)rows, kLoopThreads, 0, s>>>(xp, tgt, loss, (int)vocab, ignore_index);
     handled = true;
   }
   if (!handled) ce_loop<T><<<(unsigned)rows, kLoopThreads, 0, s>>>(xp, tgt, loss, (int)vocab, ignore_index);
@@ -762,24 +563,22 @@ static int launch_ce(const void* logits, const int64_t* tgt, float* loss, void* 
 // Last-dim reductions (reduce over a contiguous row): sum with fp32 accumulation rounded once
 // (x.sum(-1), reference.py:72-74), max exact with NaN propagation (x.max(-1).values, :76-78).
 // =============================================================================================
-template <typename T, int L, int VPT, bool MAX>
+template <typename T, int L, int VPT, bool MAX, bool ANY>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void reduce_rows(
     const typename T::S* __restrict__ x, typename T::S* __restrict__ y, int64_t rows, int cols) {
   using G = RowGeom<L>;
-  using R = RowRegs<T, L, VPT>;
+  using R = RowRegs<T, L, VPT, ANY>;
   __shared__ float red[G::kWPB];
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const int nvec = active ? cols / T::kVec : 0;
+  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
   R r;
-  r.load(x + row * cols, nvec, gl);
+  r.load(x + row * cols, sh, gl);
   float a = MAX ? -INFINITY : 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
-    if (R::valid(j, gl, nvec))
-#pragma unroll
-      for (int e = 0; e < T::kVec; ++e) a = MAX ? nan_max(a, r.f[j * T::kVec + e]) : a + r.f[j * T::kVec + e];
+    if (R::valid(j, gl, sh.nvec)) r.each(j, gl, sh, [&](float v) { a = MAX ? nan_max(a, v) : a + v; });
   a = group_reduce<L, MAX ? 2 : 0>(a, red);
   if (active && gl == 0) y[row] = T::from_f(a);
 }
@@ -964,13 +763,13 @@ static int launch_reduce(const void* x, void* y, int64_t outer, int64_t red_n, i
   if (inner == 1) {
     const int64_t rows = outer, cols = red_n;
     RowPlan plan;
-    const bool vec = cols % T::kVec == 0 && host_aligned16(x);
+    const bool any = cols % T::kVec != 0 || !host_aligned16(x);
     bool handled = false;
-    if (vec && plan_row(cols / T::kVec, T::kVec, &plan, 2)) {
-      AK_ROW_SWITCH({
+    if (plan_row_cols(cols, T::kVec, any, &plan, 2)) {
+      AK_ANY_SWITCH(any, AK_ROW_SWITCH({
         const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-        reduce_rows<T, L, VPT, MAX><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, yp, rows, (int)cols);
-      });
+        reduce_rows<T, L, VPT, MAX, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, yp, rows, (int)cols);
+      }));
     }
     if (!handled) reduce_loop<T, MAX><<<(unsigned)rows, kLoopThreads, 0, s>>>(xp, yp, (int)cols);
     return record_launch();

@@ -832,6 +832,66 @@ def test_softmax_ce_wide_odd_rows(gpu, cols, dtype):
         assert math.isnan(lr) and math.isnan(er), (cols, dtype, r, lr, er)
 
 
+@pytest.mark.parametrize("cols", [4, 7, 8, 9, 15, 63, 130, 513, 1023, 4095, 4097, 16385, 32767, 32770, 65530, 65535, 65537])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+def test_row_ops_any_width_and_alignment(gpu, cols, dt):
+    """The row ops on rows of every width class (narrower than a vector, a vector's edges, the lane and
+    register limits, past them) starting one element past an aligned address, inputs and outputs inside
+    buffers whose other elements are NaN (a read past the row would spread it) and must stay NaN (a write
+    past it would not). Against 64 bits: fp32 sums of n terms within n 2^-24 of the absolute sum, one
+    rounding (rmsnorm: four) of the result; maxima exact. Two row counts: few rows, and enough that
+    cross-entropy streams its widest rows."""
+    from autokernel_amd.kernels import _ops
+    u = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dt]
+    tiny = {torch.float16: 6e-8, torch.bfloat16: 1e-38, torch.float32: 1e-38}[dt]
+    for rows in (3, 600 if cols in (16385, 32770) else 9):
+        g = torch.Generator().manual_seed(cols + rows)
+        X, W, Bi = (torch.randn(*s, generator=g).to(dt) for s in ((rows, cols), (cols,), (cols,)))
+
+        def inside(t, off=1):
+            buf = torch.full((t.numel() + 40,), math.nan, dtype=dt, device=gpu)
+            buf[off:off + t.numel()] = t.flatten().to(gpu)
+            return buf, buf[off:off + t.numel()].view(t.shape)
+
+        def check(name, y, buf, exact, bound):
+            d = (y.double().cpu() - exact).abs()
+            assert bool((d <= bound).all()), (name, rows, cols, float((d / bound).max()))
+            assert int(torch.isnan(buf).sum()) == 40, (name, rows, cols)
+        _, x = inside(X)
+        _, w = inside(W, 3)
+        _, b = inside(Bi, 5)
+        Xd, n24 = X.double(), (cols + 16) * 2.0 ** -24
+        for off in (1, 0):
+            def out(shape):
+                return inside(torch.zeros(*shape, dtype=dt), off)
+            buf, y = out((rows, cols))
+            _ops.rmsnorm(y, x, w, 1e-6)
+            e = Xd / (Xd.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt() * W.double()
+            check("rmsnorm", y, buf, e, (5 * u + n24) * e.abs() + tiny)
+            buf, y = out((rows, cols))
+            _ops.layernorm(y, x, w, b, 1e-5)
+            mean, var = Xd.mean(-1, keepdim=True), Xd.var(-1, unbiased=False, keepdim=True)
+            h = (Xd - mean) / (var + 1e-5).sqrt() * W.double()
+            e = h + Bi.double()
+            slack = n24 * (Xd.abs().mean(-1, keepdim=True) / (var + 1e-5).sqrt() * W.double().abs() + 2 * h.abs())
+            check("layernorm", y, buf, e, u * e.abs() + 2 * slack + 8 * 2.0 ** -24 * (h.abs() + e.abs()) + tiny)
+            buf, y = out((rows, cols))
+            _ops.softmax(y, x)
+            e = Xd.softmax(-1)
+            check("softmax", y, buf, e, (u + n24 + 2.0 ** -19) * e + tiny)  # 2^-19: the exponent's rounding at |x log2 e| <= 16
+            buf, y = out((rows,))
+            _ops.reduce_sum(y, x, rows, cols, 1)
+            check("sum", y, buf, Xd.sum(-1), u * Xd.sum(-1).abs() + n24 * Xd.abs().sum(-1) + tiny)
+            buf, y = out((rows,))
+            _ops.reduce_max(y, x, rows, cols, 1)
+            check("max", y, buf, Xd.max(-1).values, tiny * torch.ones(()))
+        t = torch.randint(0, cols, (rows,), generator=g)
+        loss, o = torch.empty(rows, device=gpu), torch.empty((), device=gpu, dtype=dt)
+        _ops.cross_entropy(o, loss, x, t.to(gpu), -100)
+        e = torch.nn.functional.cross_entropy(Xd, t)
+        assert abs(float(o) - float(e)) <= (2 * u + n24 + 2.0 ** -19) * (float(e) + 6), (rows, cols, float(o), float(e))
+
+
 def test_cross_entropy_ignore_and_3d(gpu):
     g = torch.Generator().manual_seed(9)
     logits = torch.randn(2, 50, 320, generator=g).half()
