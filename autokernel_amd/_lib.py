@@ -132,10 +132,14 @@ def require_gpu(op: str, *tensors: torch.Tensor) -> None:
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def stream_of(t: torch.Tensor) -> int:
+def stream_of_index(index: int) -> int:
     if _raw_stream is not None:
-        return _raw_stream(t.get_device())
-    return torch.cuda.current_stream(t.device).cuda_stream
+        return _raw_stream(index)
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+def stream_of(t: torch.Tensor) -> int:
+    return stream_of_index(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

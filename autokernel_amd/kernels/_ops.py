@@ -9,6 +9,7 @@ that device and raises AkError on a non-OK status.
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 
 import torch
@@ -16,55 +17,58 @@ import torch
 from .. import _lib
 
 
-def _code(t: torch.Tensor, op: str) -> int:
-    return _lib.dtype_code(t, op)
+_code = _lib.dtype_code
+_I64x3 = ctypes.c_int64 * 3
 
 
-def _run(fn_name: str, ref: torch.Tensor, *args, **info) -> None:
+def _run(fn_name: str, ref: torch.Tensor, info, *args) -> None:
+    """Call fn_name(*args, stream) on ref's device. info: a function giving the error message's
+    details, called for a failed launch only: building them (shape tuples, keyword dicts) cost
+    0.7 us of every good one."""
     idx = ref.get_device()
     if idx < 0:
         raise RuntimeError(f"{fn_name}: expected GPU tensors, got one on {ref.device} (no CPU path)")
     fn = getattr(_lib.load(), fn_name)
     if idx == torch.cuda.current_device():
-        st = fn(*args, _lib.stream_of(ref))
+        st = fn(*args, _lib.stream_of_index(idx))
     else:
         with torch.cuda.device(idx):
-            st = fn(*args, _lib.stream_of(ref))
+            st = fn(*args, _lib.stream_of_index(idx))
     if st != _lib.AK_OK:
-        _lib.check(st, fn_name, **info)
+        _lib.check(st, fn_name, **info())
 
 
 def rmsnorm(y: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: float) -> None:
-    _run("ak_rmsnorm", x, _code(x, "rmsnorm"), x.data_ptr(), weight.data_ptr(), y.data_ptr(), x.shape[0],
-         x.shape[1], float(eps), shape=tuple(x.shape), dtype=x.dtype)
+    _run("ak_rmsnorm", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), _code(x, "rmsnorm"), x.data_ptr(),
+         weight.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1], float(eps))
 
 
 def rmsnorm_rsqrt(y: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: float) -> None:
-    _run("ak_rmsnorm_rsqrt", x, _code(x, "rmsnorm"), x.data_ptr(), weight.data_ptr(), y.data_ptr(),
-         x.shape[0], x.shape[1], float(eps), shape=tuple(x.shape), dtype=x.dtype)
+    _run("ak_rmsnorm_rsqrt", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), _code(x, "rmsnorm"), x.data_ptr(),
+         weight.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1], float(eps))
 
 
 def layernorm(y: torch.Tensor, x: torch.Tensor, weight: torch.Tensor | None, bias: torch.Tensor | None,
               eps: float) -> None:
-    _run("ak_layernorm", x, _code(x, "layernorm"), x.data_ptr(), _lib.ptr(weight), _lib.ptr(bias), y.data_ptr(),
-         x.shape[0], x.shape[1], float(eps), shape=tuple(x.shape), dtype=x.dtype)
+    _run("ak_layernorm", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), _code(x, "layernorm"), x.data_ptr(),
+         _lib.ptr(weight), _lib.ptr(bias), y.data_ptr(), x.shape[0], x.shape[1], float(eps))
 
 
 def softmax(y: torch.Tensor, x: torch.Tensor) -> None:
-    _run("ak_softmax", x, _code(x, "softmax"), x.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1],
-         shape=tuple(x.shape), dtype=x.dtype)
+    _run("ak_softmax", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), _code(x, "softmax"), x.data_ptr(),
+         y.data_ptr(), x.shape[0], x.shape[1])
 
 
 def rope(y: torch.Tensor, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, rep_inner: int) -> None:
-    _run("ak_rope", x, _code(x, "rotary_embedding"), x.data_ptr(), cos.data_ptr(), sin.data_ptr(), y.data_ptr(),
-         x.shape[0], x.shape[1], cos.shape[0], int(rep_inner), shape=tuple(x.shape), dtype=x.dtype)
+    _run("ak_rope", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), _code(x, "rotary_embedding"), x.data_ptr(),
+         cos.data_ptr(), sin.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1], cos.shape[0], int(rep_inner))
 
 
 def cross_entropy(out: torch.Tensor, row_loss: torch.Tensor, logits: torch.Tensor, targets: torch.Tensor,
                   ignore_index: int) -> None:
-    _run("ak_cross_entropy", logits, _code(logits, "cross_entropy"), logits.data_ptr(), targets.data_ptr(),
-         row_loss.data_ptr(), out.data_ptr(), logits.shape[0], logits.shape[1], int(ignore_index),
-         shape=tuple(logits.shape), dtype=logits.dtype)
+    _run("ak_cross_entropy", logits, lambda: dict(shape=tuple(logits.shape), dtype=logits.dtype),
+         _code(logits, "cross_entropy"), logits.data_ptr(), targets.data_ptr(), row_loss.data_ptr(), out.data_ptr(),
+         logits.shape[0], logits.shape[1], int(ignore_index))
 
 
 @functools.lru_cache(maxsize=1024)
@@ -78,10 +82,11 @@ def _reduce(name: str, y: torch.Tensor, x: torch.Tensor, outer: int, reduce: int
     nbytes = _reduce_workspace_bytes(code, outer, reduce, inner) if inner > 1 else 0
     if nbytes > 0:  # fp32 partial sums of row slices
         ws = torch.empty(nbytes // 4, device=x.device, dtype=torch.float32)
-        _run(f"ak_{name}_ws", x, code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, ws.data_ptr(), nbytes,
-             shape=tuple(x.shape), dtype=x.dtype)
+        _run(f"ak_{name}_ws", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), code, x.data_ptr(), y.data_ptr(),
+             outer, reduce, inner, ws.data_ptr(), nbytes)
         return
-    _run(f"ak_{name}", x, code, x.data_ptr(), y.data_ptr(), outer, reduce, inner, shape=tuple(x.shape), dtype=x.dtype)
+    _run(f"ak_{name}", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), code, x.data_ptr(), y.data_ptr(), outer,
+         reduce, inner)
 
 
 def reduce_sum(y: torch.Tensor, x: torch.Tensor, outer: int, reduce: int, inner: int) -> None:
@@ -104,12 +109,12 @@ def gemm(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, b_trans: bool,
     N = b.shape[0] if b_trans else b.shape[1]
     code = _code(a, "matmul")
     if workspace is not None and workspace.numel() > 0:
-        _run("ak_gemm_ws", a, code, a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c),
-             int(bool(b_trans)), workspace.data_ptr(), workspace.numel() * 4, M=M, N=N, K=K, b_trans=b_trans,
-             dtype=a.dtype)
+        _run("ak_gemm_ws", a, lambda: dict(M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype), code, a.data_ptr(),
+             b.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c), int(bool(b_trans)), workspace.data_ptr(),
+             workspace.numel() * 4)
         return
-    _run("ak_gemm", a, code, a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c),
-         int(bool(b_trans)), M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype)
+    _run("ak_gemm", a, lambda: dict(M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype), code, a.data_ptr(), b.data_ptr(),
+         c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c), int(bool(b_trans)))
 
 
 def gemm_batched(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, b_trans: bool) -> None:
@@ -120,26 +125,27 @@ def gemm_batched(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, b_trans: boo
 
     def ld(t):
         return t.stride(1) if t.shape[1] > 1 else max(t.shape[2], 1)
-    _run("ak_gemm_batched", a, _code(a, "matmul"), a.data_ptr(), b.data_ptr(), c.data_ptr(), Z, M, N, K, ld(a),
-         ld(b), ld(c), a.stride(0), b.stride(0), c.stride(0), int(bool(b_trans)), Z=Z, M=M, N=N, K=K,
-         b_trans=b_trans, dtype=a.dtype)
+    _run("ak_gemm_batched", a, lambda: dict(Z=Z, M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype), _code(a, "matmul"),
+         a.data_ptr(), b.data_ptr(), c.data_ptr(), Z, M, N, K, ld(a), ld(b), ld(c), a.stride(0), b.stride(0),
+         c.stride(0), int(bool(b_trans)))
 
 
 def gemm_bias(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor, b_trans: bool) -> None:
     """c = a @ op(b) + bias [N], the bias added to the fp32 accumulator (one rounding)."""
     M, K = a.shape
     N = b.shape[0] if b_trans else b.shape[1]
-    _run("ak_gemm_bias", a, _code(a, "gemm_bias"), a.data_ptr(), b.data_ptr(), bias.data_ptr(), c.data_ptr(), M, N, K,
-         _ld(a), _ld(b), _ld(c), int(bool(b_trans)), M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype)
+    _run("ak_gemm_bias", a, lambda: dict(M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype), _code(a, "gemm_bias"),
+         a.data_ptr(), b.data_ptr(), bias.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c),
+         int(bool(b_trans)))
 
 
 def gemm_bias_gelu(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor, b_trans: bool) -> None:
     """c = gelu(a @ op(b) + bias): the biased product rounded, then exact GELU, rounded again."""
     M, K = a.shape
     N = b.shape[0] if b_trans else b.shape[1]
-    _run("ak_gemm_bias_gelu", a, _code(a, "gemm_bias_gelu"), a.data_ptr(), b.data_ptr(), bias.data_ptr(),
-         c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c), int(bool(b_trans)), M=M, N=N, K=K, b_trans=b_trans,
-         dtype=a.dtype)
+    _run("ak_gemm_bias_gelu", a, lambda: dict(M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype),
+         _code(a, "gemm_bias_gelu"), a.data_ptr(), b.data_ptr(), bias.data_ptr(), c.data_ptr(), M, N, K, _ld(a),
+         _ld(b), _ld(c), int(bool(b_trans)))
 
 
 def gemm_bias_residual(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor, r: torch.Tensor,
@@ -147,17 +153,29 @@ def gemm_bias_residual(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, bias: 
     """c = r + (a @ op(b) + bias): the biased product rounded, then the sum (r shares c's row stride)."""
     M, K = a.shape
     N = b.shape[0] if b_trans else b.shape[1]
-    _run("ak_gemm_bias_residual", a, _code(a, "gemm_bias_residual"), a.data_ptr(), b.data_ptr(), bias.data_ptr(),
-         r.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c), int(bool(b_trans)), M=M, N=N, K=K,
-         b_trans=b_trans, dtype=a.dtype)
+    _run("ak_gemm_bias_residual", a, lambda: dict(M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype),
+         _code(a, "gemm_bias_residual"), a.data_ptr(), b.data_ptr(), bias.data_ptr(), r.data_ptr(), c.data_ptr(), M,
+         N, K, _ld(a), _ld(b), _ld(c), int(bool(b_trans)))
 
 
 def gemm_residual(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, r: torch.Tensor, b_trans: bool) -> None:
     """c = r + a @ op(b), the product rounded, then the sum (r shares c's row stride)."""
     M, K = a.shape
     N = b.shape[0] if b_trans else b.shape[1]
-    _run("ak_gemm_residual", a, _code(a, "gemm_residual"), a.data_ptr(), b.data_ptr(), r.data_ptr(), c.data_ptr(),
-         M, N, K, _ld(a), _ld(b), _ld(c), int(bool(b_trans)), M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype)
+    _run("ak_gemm_residual", a, lambda: dict(M=M, N=N, K=K, b_trans=b_trans, dtype=a.dtype),
+         _code(a, "gemm_residual"), a.data_ptr(), b.data_ptr(), r.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b),
+         _ld(c), int(bool(b_trans)))
+
+
+def linear(c: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, r: torch.Tensor | None,
+           gelu: bool, M: int, N: int, K: int) -> None:
+    """gemm_bias, gemm_bias_gelu, gemm_bias_residual or gemm_residual (whichever bias, r and gelu
+    name) of dense x [.., K] (M rows), w [N, K], bias [N], r and c [.., N], whatever their rank."""
+    name, mid = (("ak_gemm_residual", (r.data_ptr(),)) if bias is None
+                 else ("ak_gemm_bias_residual", (bias.data_ptr(), r.data_ptr())) if r is not None
+                 else ("ak_gemm_bias_gelu" if gelu else "ak_gemm_bias", (bias.data_ptr(),)))
+    _run(name, x, lambda: dict(M=M, N=N, K=K, b_trans=True, dtype=x.dtype), _code(x, "linear"), x.data_ptr(),
+         w.data_ptr(), *mid, c.data_ptr(), M, N, K, K, K, max(N, 1), 1)
 
 
 def gemm_rope(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, b_trans: bool, cos: torch.Tensor, sin: torch.Tensor,
@@ -165,17 +183,18 @@ def gemm_rope(c: torch.Tensor, a: torch.Tensor, b: torch.Tensor, b_trans: bool, 
     """c = a @ op(b) with the model's rotary embedding on columns [0, rot_cols) (fp32 tables)."""
     M, K = a.shape
     N = b.shape[0] if b_trans else b.shape[1]
-    _run("ak_gemm_rope", a, _code(a, "gemm_rope"), a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b),
-         _ld(c), int(bool(b_trans)), cos.data_ptr(), sin.data_ptr(), seq_len, head_dim, rot_cols, M=M, N=N, K=K,
-         head_dim=head_dim, rot_cols=rot_cols, dtype=a.dtype)
+    _run("ak_gemm_rope", a, lambda: dict(M=M, N=N, K=K, head_dim=head_dim, rot_cols=rot_cols, dtype=a.dtype),
+         _code(a, "gemm_rope"), a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, _ld(a), _ld(b), _ld(c),
+         int(bool(b_trans)), cos.data_ptr(), sin.data_ptr(), seq_len, head_dim, rot_cols)
 
 
 def rope_f32_tables(y: torch.Tensor, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, rows: int, head_dim: int,
                     table_rows: int, rep_inner: int, x_tok_stride: int) -> None:
     """The model's RoPE: x (rows / rep_inner tokens of rep_inner heads, token stride x_tok_stride)
     rotated by fp32 tables into dense y."""
-    _run("ak_rope_f32_tables", x, _code(x, "rope_f32_tables"), x.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-         y.data_ptr(), rows, head_dim, table_rows, rep_inner, x_tok_stride, shape=tuple(x.shape), dtype=x.dtype)
+    _run("ak_rope_f32_tables", x, lambda: dict(shape=tuple(x.shape), dtype=x.dtype), _code(x, "rope_f32_tables"),
+         x.data_ptr(), cos.data_ptr(), sin.data_ptr(), y.data_ptr(), rows, head_dim, table_rows, rep_inner,
+         x_tok_stride)
 
 
 @functools.lru_cache(maxsize=1024)
@@ -187,8 +206,8 @@ def gemm_workspace_bytes(dtype: int, M: int, N: int, K: int, lda: int, ldb: int,
 def mlp_gate_up(h: torch.Tensor, x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, activation: int) -> None:
     M, D = x.shape
     H = w_gate.shape[0]
-    _run("ak_mlp_gate_up", x, _code(x, "fused_mlp"), x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), h.data_ptr(),
-         M, H, D, int(activation), M=M, H=H, D=D, dtype=x.dtype)
+    _run("ak_mlp_gate_up", x, lambda: dict(M=M, H=H, D=D, dtype=x.dtype), _code(x, "fused_mlp"), x.data_ptr(),
+         w_gate.data_ptr(), w_up.data_ptr(), h.data_ptr(), M, H, D, int(activation))
 
 
 @functools.lru_cache(maxsize=1024)
@@ -201,16 +220,16 @@ def flash_attn_fwd(o: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.T
     """Q, O [B, Hq, Sq, D], K, V [B, Hkv, Sk, D], any strides with a contiguous head_dim."""
     B, Hq, Sq, D = q.shape
     Hkv, Sk = k.shape[1], k.shape[2]
-    st = [_lib.i64_array(t.stride()[:3]) for t in (q, k, v, o)]
+    st = [_I64x3(*t.stride()[:3]) for t in (q, k, v, o)]
     code = _code(q, "flash_attention")
     # fp32 partials of key slices: only calls with few query rows per KV head have any
     nbytes = _attn_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, bool(causal)) if Sq <= 16 else 0
     if nbytes > 0:
         ws = torch.empty(nbytes // 4, device=q.device, dtype=torch.float32)
-        _run("ak_flash_attn_fwd_ws", q, code, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, Hq, Hkv, Sq,
-             Sk, D, st[0], st[1], st[2], st[3], int(bool(causal)), float(sm_scale), ws.data_ptr(), nbytes,
-             Q=tuple(q.shape), K=tuple(k.shape), dtype=q.dtype)
+        _run("ak_flash_attn_fwd_ws", q, lambda: dict(Q=tuple(q.shape), K=tuple(k.shape), dtype=q.dtype), code,
+             q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, Hq, Hkv, Sq, Sk, D, st[0], st[1], st[2],
+             st[3], int(bool(causal)), float(sm_scale), ws.data_ptr(), nbytes)
         return
-    _run("ak_flash_attn_fwd", q, code, q.data_ptr(), k.data_ptr(), v.data_ptr(),
-         o.data_ptr(), B, Hq, Hkv, Sq, Sk, D, st[0], st[1], st[2], st[3], int(bool(causal)), float(sm_scale),
-         Q=tuple(q.shape), K=tuple(k.shape), dtype=q.dtype)
+    _run("ak_flash_attn_fwd", q, lambda: dict(Q=tuple(q.shape), K=tuple(k.shape), dtype=q.dtype), code, q.data_ptr(),
+         k.data_ptr(), v.data_ptr(), o.data_ptr(), B, Hq, Hkv, Sq, Sk, D, st[0], st[1], st[2], st[3],
+         int(bool(causal)), float(sm_scale))

@@ -17,15 +17,10 @@ from __future__ import annotations
 import torch
 
 from . import _ops
+from .host import _attn_operand as _prep
 from .host import flash_attention as kernel_fn  # noqa: F401
 
 KERNEL_TYPE = "flash_attention"
-
-
-def _prep(t: torch.Tensor) -> torch.Tensor:
-    if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]) or t.data_ptr() % 16:
-        t = t.contiguous()
-    return t
 
 
 def attention(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, causal: bool = True,

@@ -7,7 +7,8 @@ instead of copying; a row-major [K, N] B is read in place too (b_trans = 0). Run
 (gemm.hip), or, for kernel_fn, ak_gemm_ws with a torch-allocated fp32 workspace when few output tiles
 and a long K would leave most CUs idle (K split into slices that run side by side, then added in a
 fixed order). kernel_fn is kernels/host.py's matmul; gemm, gemm_bias, gemm_bias_gelu, gemm_bias_residual,
-gemm_residual and gemm_rope are the 2-D forms (and fused epilogues) the model plug-in uses.
+gemm_residual and gemm_rope are the 2-D forms (and fused epilogues) the model plug-in uses, linear
+their form on a Linear's own input and weight.
 """
 from __future__ import annotations
 
@@ -107,6 +108,41 @@ def gemm_residual(A: torch.Tensor, B: torch.Tensor, R: torch.Tensor) -> torch.Te
         raise ValueError(f"gemm_residual: R {tuple(R.shape)} {R.dtype} does not fit [{M}, {N}] {A.dtype}")
     C = torch.empty((M, N), device=A.device, dtype=A.dtype)
     _ops.gemm_residual(C, A, Bs, R.contiguous(), bt)
+    return C
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
+           residual: torch.Tensor | None = None, gelu: bool = False) -> torch.Tensor:
+    """A Linear on x [..., K] with its weight as stored, [N, K]: gemm_bias, gemm_bias_gelu (gelu),
+    gemm_bias_residual or gemm_residual of x's rows, in x's leading shape (with a residual: in its
+    shape). Dense operands go to the same entry point without the view calls around it, which took
+    3 of the 13 us of a small Linear; everything else goes through those functions."""
+    op = "linear"
+    if gelu and (bias is None or residual is not None):
+        raise ValueError(f"{op}: gelu needs a bias and no residual")
+    K, N = x.shape[-1], weight.shape[0]
+    dense = K > 1 and weight.dim() == 2 and x.is_contiguous() and weight.is_contiguous() and (
+        residual is None or residual.is_contiguous())
+    if not dense or (bias is None and residual is None):
+        A, B = x.reshape(-1, K), weight.t()
+        r2 = None if residual is None else residual.reshape(-1, residual.shape[-1])
+        if residual is None:
+            C = gemm(A, B) if bias is None else (gemm_bias_gelu if gelu else gemm_bias)(A, B, bias)
+            return C.view(*x.shape[:-1], N)
+        C = gemm_residual(A, B, r2) if bias is None else gemm_bias_residual(A, B, bias, r2)
+        return C.view(residual.shape)
+    M = x.numel() // K
+    if weight.shape[1] != K:
+        raise ValueError(f"{op}: x {tuple(x.shape)} does not fit weight {tuple(weight.shape)}")
+    if x.dtype != weight.dtype or x.dtype not in (torch.float16, torch.bfloat16):
+        raise ValueError(f"{op}: needs one f16 / bf16 dtype, got {x.dtype}, {weight.dtype}")
+    host._check(op, x, weight)
+    if bias is not None:
+        bias = _bias_operand(op, bias, x, N)
+    if residual is not None and (residual.shape[-1] != N or residual.numel() != M * N or residual.dtype != x.dtype):
+        raise ValueError(f"{op}: residual {tuple(residual.shape)} {residual.dtype} does not fit [{M}, {N}] {x.dtype}")
+    C = torch.empty(x.shape[:-1] + (N,) if residual is None else residual.shape, device=x.device, dtype=x.dtype)
+    _ops.linear(C, x, weight, bias, residual, gelu, M, N, K)
     return C
 
 

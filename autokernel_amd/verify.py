@@ -52,7 +52,7 @@ from . import kernels
 from .kernels import flash_attention as fa_mod
 from .kernels import rotary_embedding as rope_mod
 from .kernels.fused_mlp import gate_up
-from .kernels.matmul import gemm, gemm_bias, gemm_bias_gelu, gemm_bias_residual, gemm_residual, gemm_rope
+from .kernels.matmul import gemm, gemm_rope, linear
 from .kernels.rmsnorm import rms_norm_rsqrt
 
 ALL_KERNELS = ("matmul", "rmsnorm", "layernorm", "rotary_embedding", "flash_attention", "fused_mlp")
@@ -218,14 +218,9 @@ MODULE_WRAPPERS = {"matmul": ModuleLinearWrapper, "layernorm": ModuleLayerNormWr
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x @ W.T (+ bias) with W read in place; an f16 / bf16 bias is fused into the GEMM and
     rounded once with the product, as stock nn.Linear (addmm) rounds it."""
-    x2 = x.reshape(-1, x.shape[-1])
-    if bias is not None and bias.dtype == x.dtype and x.dtype in (torch.float16, torch.bfloat16):
-        out = gemm_bias(x2, weight.t(), bias)
-    else:
-        out = gemm(x2, weight.t())
-        if bias is not None:
-            out = out + bias
-    return out.view(*x.shape[:-1], weight.shape[0])
+    if bias is None or bias.dtype == x.dtype and x.dtype in (torch.float16, torch.bfloat16):
+        return linear(x, weight, bias)
+    return (gemm(x.reshape(-1, x.shape[-1]), weight.t()) + bias).view(*x.shape[:-1], weight.shape[0])
 
 
 class LinearWrapper(nn.Module):
@@ -284,8 +279,7 @@ class FeedForwardWrapper(nn.Module):
             return y if residual is None else residual + y
         x2 = x.reshape(-1, x.shape[-1]).contiguous()
         h = gate_up(x2, self.gate.weight, self.up.weight, "silu")
-        y = gemm_residual(h, self.down.weight.t(), residual.reshape(-1, residual.shape[-1]))
-        return y.view(residual.shape)
+        return linear(h, self.down.weight, None, residual)
 
 
 def _fusable(residual: torch.Tensor) -> bool:
@@ -308,12 +302,8 @@ def _linear_residual(x: torch.Tensor, lin: nn.Linear, residual: Optional[torch.T
     product (+ bias) is rounded, then the sum, as the separate add rounds it."""
     if residual is None:
         return _linear(x, lin.weight, lin.bias)
-    x2 = x.reshape(-1, x.shape[-1])
-    r2 = residual.reshape(-1, residual.shape[-1])
-    if _bias_fusable(lin, x):
-        return gemm_bias_residual(x2, lin.weight.t(), lin.bias, r2).view(residual.shape)
-    if lin.bias is None and _fusable(x):
-        return gemm_residual(x2, lin.weight.t(), r2).view(residual.shape)
+    if _bias_fusable(lin, x) or (lin.bias is None and _fusable(x)):
+        return linear(x, lin.weight, lin.bias, residual)
     return residual + _linear(x, lin.weight, lin.bias)
 
 
@@ -338,8 +328,7 @@ class GeluMLPWrapper(nn.Module):
             y = _linear(self.gelu(_linear(x, fc.weight, fc.bias)), proj.weight, proj.bias)
             y = self.drop(y) if self.drop is not None else y
             return y if residual is None else residual + y
-        h = gemm_bias_gelu(x.reshape(-1, x.shape[-1]), fc.weight.t(), fc.bias)
-        return _linear_residual(h.view(*x.shape[:-1], -1), proj, residual)
+        return _linear_residual(linear(x, fc.weight, fc.bias, gelu=True), proj, residual)
 
 
 def _rope_tables_from(args) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -452,8 +441,7 @@ class AttentionWrapper(nn.Module):
         if residual is None:
             return self._proj(o.wo, y)
         if self.use_matmul and o.wo.bias is None and _fusable(residual):
-            out = gemm_residual(y.reshape(B * T, H * D), o.wo.weight.t(), residual.reshape(B * T, -1))
-            return out.view(residual.shape)
+            return linear(y, o.wo.weight, None, residual)
         return residual + self._proj(o.wo, y)
 
 
@@ -502,7 +490,7 @@ class EncoderAttentionWrapper(nn.Module):
             return _linear(t, lin.weight, lin.bias) if self.use_matmul else lin(t)
         if self.fused_qkv:
             qkv = _linear(x, *self._qkv_params())
-            q, k, v = (qkv[..., i * C:(i + 1) * C].view(B, T, H, D) for i in range(3))
+            q, k, v = qkv.view(B, T, 3, H, D).unbind(2)
         else:
             q, k, v = (proj(lin, x).view(B, T, H, D) for lin in (o.query, o.key, o.value))
         y = torch.empty((B, T, H, D), device=x.device, dtype=x.dtype)  # written in place, no transpose copy
@@ -536,7 +524,7 @@ class FusedQKVAttentionWrapper(nn.Module):
         def proj(lin, t):
             return _linear(t, lin.weight, lin.bias) if self.use_matmul else lin(t)
         qkv = proj(o.c_attn, x)
-        q, k, v = (qkv[..., i * C:(i + 1) * C].view(B, T, H, D).transpose(1, 2) for i in range(3))
+        q, k, v = qkv.view(B, T, 3, H, D).permute(2, 0, 3, 1, 4).unbind(0)  # column slices, [B, H, T, D] each
         y = torch.empty((B, T, H, D), device=x.device, dtype=x.dtype)  # written in place, no transpose copy
         fa_mod.attention(q, k, v, True, None, out=y.transpose(1, 2))
         y = y.view(B, T, C)

@@ -1206,6 +1206,37 @@ def test_gemm_bias_gelu_and_residual_epilogues(gpu, M, N, K):
         print(f"gemm bias+residual {M}x{N}x{K} {dt}: bit-equal", flush=True)
 
 
+@pytest.mark.parametrize("lead,N,K", [((3,), 96, 64), ((2, 5), 72, 40), ((1, 1, 130), 136, 256), ((4, 0), 64, 64),
+                                      ((), 33, 24), ((7, 9), 1, 64), ((65,), 80, 1)])
+def test_linear_equals_gemm_forms(gpu, lead, N, K):
+    """linear (the stored weight read in place, any leading shape, no views) gives the bits, shape and
+    strides of the gemm form it stands for, dense and strided, with each of bias, GELU and residual;
+    what does not fit is refused."""
+    from autokernel_amd.kernels import matmul as mm
+    for dt in (torch.float16, torch.bfloat16):
+        g = torch.Generator().manual_seed(N + K)
+        wide = torch.randn(*lead, K + 8, generator=g).to(dt).to(gpu)
+        W = (torch.randn(N, K, generator=g) * 0.1).to(dt).to(gpu)
+        b, r = torch.randn(N, generator=g).to(dt).to(gpu), torch.randn(*lead, N, generator=g).to(dt).to(gpu)
+        for x in (wide[..., 8:], wide[..., 8:].contiguous()):
+            x2, r2 = x.reshape(-1, K), r.reshape(-1, N)
+            for out, want in ((mm.linear(x, W), mm.gemm(x2, W.t())),
+                              (mm.linear(x, W, b), mm.gemm_bias(x2, W.t(), b)),
+                              (mm.linear(x, W, b, gelu=True), mm.gemm_bias_gelu(x2, W.t(), b)),
+                              (mm.linear(x, W, b, r), mm.gemm_bias_residual(x2, W.t(), b, r2)),
+                              (mm.linear(x, W, None, r), mm.gemm_residual(x2, W.t(), r2))):
+                want = want.view(*lead, N)
+                assert torch.equal(out, want) and out.stride() == want.stride(), (lead, N, K, dt)
+        with pytest.raises(ValueError):
+            mm.linear(x, W, b.float())
+        with pytest.raises(ValueError):
+            mm.linear(x, W, b, r[..., :-1] if N > 1 else r.float())
+        with pytest.raises(ValueError):
+            mm.linear(x, W.float(), b)
+        with pytest.raises(ValueError):
+            mm.linear(x, W, None, gelu=True)
+
+
 def test_gemm_bias_gelu_every_value(gpu):
     """Every finite f16 / bf16 value through ak_gemm_bias_gelu once: with A the [256, 256] identity
     and a zero bias, C[m, n] = W[n, m] exactly, so W [N, 256] holding all finite values feeds each
