@@ -418,8 +418,8 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
   wait_vmcnt<0>();  // no DMA may still target this block's LDS when its waves end
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int MF>
-__global__ __launch_bounds__(WM* WN* kWave) void gemm_dma(
+template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int MF, int OCC>
+__global__ __launch_bounds__(WM* WN* kWave, OCC* WM* WN / 4) void gemm_dma(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
     uint16_t* __restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
     int tiles_m, int tiles_n, EpiArgs ep) {
@@ -512,22 +512,29 @@ struct TileCfg {
 // launch, weighted by the per-tile efficiency of smaller tiles (more LDS and L2 traffic per flop).
 // wide192: also consider 256x192 tiles (the LDS-DMA kernel with nn.Linear-layout B; 2048 x 6144,
 // a fused QKV projection, is then exactly one tile per CU). small64: also consider 64x64 tiles
-// (the same kernel, for grids that 128x128 tiles leave mostly idle).
+// (the same kernel, for grids that 128x128 tiles leave mostly idle) and 64x128 ones, and, with
+// nn.Linear-layout B, 64x96 and 128x192 (whose weight is eff192, see kPairK).
 static TileCfg pick_tile(int64_t M, int64_t N, int nb, bool wide192 = false, bool small64 = false,
-                         int64_t batch = 1) {
-  const TileCfg cands[] = {{256, 256}, {256, 128}, {128, 128}, {256, 192}, {64, 64}};
+                         int64_t batch = 1, double eff192 = 0.0) {
+  const TileCfg cands[] = {{256, 256}, {256, 128}, {128, 128}, {256, 192}, {64, 64}, {128, 192}, {64, 96}, {64, 128}};
   // relative per-flop throughput of the tiles (bf16, MI355X): 4096^3 on 256x256 1230 TF/s,
   // 2048x4096x4096 on 256x128 1084 TF/s, 2048x6144x4096 on 128x128 786 TF/s, on 256x192 1108 TF/s;
   // 64x64 weighted so that it wins only where 128x128 tiles fill under a third of the CUs (cold,
   // f16: 2048x768x768 16.4 -> 13.8 us, 2048x768x3072 41.7 -> 37.3 us, 1024^3 NN 17.3 -> 15.5 us,
   // 4096x768x768 unchanged at 15.1 us; with a weight of 0.5 it was also picked there and took
   // 16.3 us)
-  const double eff[] = {1.0, 0.88, 0.64, 0.88, 0.35};
+  // 64x96 and 64x128 lie between, by what a k-step of one tile on a CU takes (64x64 0.30 us, 64x96
+  // 0.36, 64x128 0.44, 128x128 0.65, 128x192 0.80, 256x128 0.97), and win where they are what fills the
+  // CUs (f16, NT, rotating operands, us, before / after): 2048x768x3072 28.1 / 21.9, 2048x768x768
+  // 11.2 / 9.6, 512x2304x768 7.8 / 6.3 (64x96), 2048x1024x4096 34.1 / 28.7, 512x4096x4096 35.1 / 28.9
+  // (64x128), 512x11008x4096 57.7 / 52.3 (128x192)
+  const double eff[] = {1.0, 0.88, 0.64, 0.88, 0.35, eff192, 0.43, 0.47};
   const int cus = 256;
   TileCfg best = cands[2];
   double best_s = -1.0;
-  for (int i = 0; i < 5; ++i) {
-    if ((i == 3 && !(wide192 && nb == 1)) || (i == 4 && !(small64 && nb == 1))) continue;
+  for (int i = 0; i < 8; ++i) {
+    const bool considered = i < 3 || (nb == 1 && (i == 3 ? wide192 : i == 5 ? eff192 > 0.0 : i == 6 ? small64 && wide192 : small64));
+    if (!considered) continue;
     const int bn = cands[i].bn / (nb == 2 ? 2 : 1);
     const int64_t tiles = cdiv(M, cands[i].bm) * cdiv(N, bn) * batch;
     const int64_t waves = cdiv(tiles, cus);
@@ -579,13 +586,14 @@ static void launch_gemm_tiled(const void* A, const void* B0, const void* B1, voi
 
 constexpr int kCUs = 256;  // MI355X compute units
 
-template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN>
+// OCC: blocks that must fit on a CU together (it bounds the registers; LDS has to fit as well).
+template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int OCC = 1>
 static void launch_dma_kernel(const void* A, const void* B0, const void* B1, void* C, int M, int N, int K,
                               int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n, hipStream_t s,
                               const EpiArgs& ep) {
   // MFMA shape 16x16x32 (32x32x16 fragments measured 4-10 % slower on every workload)
   constexpr int MF = 16;
-  gemm_dma<T, BM, BN, WM, WN, NB, EPI, BKD, NS, BKN, MF><<<dim3(tiles_m * tiles_n, ep.splits, ep.batch), WM * WN * kWave, 0, s>>>(
+  gemm_dma<T, BM, BN, WM, WN, NB, EPI, BKD, NS, BKN, MF, OCC><<<dim3(tiles_m * tiles_n, ep.splits, ep.batch), WM * WN * kWave, 0, s>>>(
       (const uint16_t*)A, (const uint16_t*)B0, (const uint16_t*)B1, (uint16_t*)C, M, N, K, lda, ldb, ldc,
       tiles_m, tiles_n, ep);
 }
@@ -606,10 +614,10 @@ struct DmaPlan {
   // Three 64-deep stages where they fit beside 8 waves, else two. Measured (bf16, NT):
   // 2048x4096x4096 on 256x128 tiles 83.5 us two-stage -> 63.4 us three-stage; 4096^3 on 256x256
   // 107.4 us two-stage (four 32-deep stages: 121.2 us, the doubled barrier count outweighs the
-  // deeper queue). The 64x64 tile (4 waves, 16 KB stages, picked for grids that larger tiles leave
-  // mostly idle) waits on transfer latency, not MFMAs: four stages keep three tiles in flight
-  // (cold, f16: 1024^3 15.5 -> 10.8 us, 2048x768x3072 37.0 -> 29.8 us, 2048x1024x1024 16.6 ->
-  // 14.6 us; four stages on 128x128 tiles gained nothing).
+  // deeper queue). The tiles of 64 rows (4 waves, 16 - 24 KB stages, picked for grids that larger
+  // tiles leave mostly idle) wait on transfer latency, not MFMAs: four stages keep three tiles in
+  // flight (cold, f16, 64x64: 1024^3 15.5 -> 10.8 us, 2048x768x3072 37.0 -> 29.8 us, 2048x1024x1024
+  // 16.6 -> 14.6 us; six or eight stages, or four on 128x128 tiles, gained nothing).
   static constexpr int BKD = 64;
   static constexpr int NS = BM == 64 ? 4 : (kFit64 >= 3 && NW == 8) ? 3 : 2;
 };
@@ -623,7 +631,9 @@ static void launch_dma_cfg(const void* A, const void* B0, const void* B1, void* 
   // then exposed; measured 2048x1024x4096: 50.9 us against 59.0 us two-stage). With more tiles the
   // 64-deep pair is faster per tile (2048x6144x4096 on 192 tiles of 256x256: 109.9 us against
   // 127.5 us).
-  constexpr bool kOk32 = P::kOk32;
+  // 64x64 tiles keep their four 64-deep stages there (f16: 128x768x768 7.3 us 32-deep, 6.3 64-deep;
+  // 512x768x3072 23.1, 17.4).
+  constexpr bool kOk32 = P::kOk32 && BM > 64;
   if (kOk32 && 2 * tiles_m * tiles_n * ep.splits * ep.batch <= kCUs) {
     if constexpr (kOk32)
       launch_dma_kernel<T, BM, BN, WM, WN, NB, EPI, 32, 4, BKN>(A, B0, B1, C, M, N, K, lda, ldb, ldc, tiles_m,
@@ -634,12 +644,49 @@ static void launch_dma_cfg(const void* A, const void* B0, const void* B1, void* 
                                                                     tiles_n, s, ep);
 }
 
+// Largest K for which 128x192 tiles are considered. A product of few k-steps spends about as long in
+// each tile's first loads and in its epilogue (bias, GELU, residual, stores) as in its MFMAs, and the
+// larger tiles have the CU to themselves, so nothing runs meanwhile. Two blocks of 8 waves and two
+// 40 KB stages share a CU, and one multiplies while the other stores. Measured (f16, NT, rotating
+// operands, us, before / after): 2048x3072x768 + GELU 25.0 / 21.0, 8192x3072x768 + GELU 75.8 / 61.4,
+// 2048x2304x768 15.2 / 13.8, 8192x2304x768 42.6 / 36.0, 8192x768x768 + residual 20.4 / 18.7,
+// 1000x5000x1024 17.0 / 16.2. A long K hides both ends and wants the larger tile's fewer LDS reads
+// per flop (8192x768x3072 53.8 / 55.0, 4096x11008x4096 317 / 350): there a 128x192 tile has the CU and
+// three stages to itself and is picked where it is what fills the chip.
+// Their weight among pick_tile's lies where they are level with the others: 256x192 tiles of which
+// every CU gets one (4096x3072x768 + bias 26.1 us as pairs, 24.1; 4096x2304x768 + bias 23.4, 22.5)
+// stay, except under the GELU, whose 50 instructions an output the pair hides (4096x3072x768 + GELU
+// 33.2, 34.9); 1024x2304x768 stays on 128x128 tiles (13.3, 9.2).
+constexpr int kPairK = 1024;
+template <int EPI>
+constexpr double kPairEff = EPI == kEpiBiasGelu ? 0.9 : 0.86;
+constexpr double kLongEff192 = 0.77;
+
 template <typename T, int NB, int EPI, bool BKN>
 static void launch_gemm_dma(const void* A, const void* B0, const void* B1, void* C, int M, int N, int K,
                             int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, const EpiArgs& ep) {
   // 256x192 needs [N, K] B: a [K, N] B tile row of 192 elements does not split into 1 KB transfers
-  const TileCfg t = pick_tile(M, N, NB, !BKN, EPI != kEpiPartial, ep.batch);
+  constexpr bool kPair = NB == 1 && !BKN && EPI != kEpiPartial;
+  const TileCfg t = pick_tile(M, N, NB, !BKN, EPI != kEpiPartial, ep.batch, !kPair ? 0.0 : K <= kPairK ? kPairEff<EPI> : kLongEff192);
   if constexpr (NB == 1) {
+    if constexpr (kPair) {
+      if (t.bm == 128 && t.bn == 192) {
+        const int tm = (int)cdiv(M, 128), tn = (int)cdiv(N, 192);
+        if (K <= kPairK) launch_dma_kernel<T, 128, 192, 2, 4, 1, EPI, 64, 2, false, 2>(A, B0, B1, C, M, N, K, lda, ldb, ldc, tm, tn, s, ep);
+        else launch_dma_kernel<T, 128, 192, 2, 4, 1, EPI, 64, 3, false>(A, B0, B1, C, M, N, K, lda, ldb, ldc, tm, tn, s, ep);
+        return;
+      }
+      if (t.bm == 64 && t.bn == 96) {
+        launch_dma_cfg<T, 64, 96, 2, 2, 1, EPI, false>(A, B0, B1, C, M, N, K, lda, ldb, ldc, s, ep);
+        return;
+      }
+    }
+    if constexpr (EPI != kEpiPartial) {
+      if (t.bm == 64 && t.bn == 128) {
+        launch_dma_cfg<T, 64, 128, 2, 2, 1, EPI, BKN>(A, B0, B1, C, M, N, K, lda, ldb, ldc, s, ep);
+        return;
+      }
+    }
     if constexpr (!BKN) {
       if (t.bm == 256 && t.bn == 192) {
         launch_dma_cfg<T, 256, 192, 2, 4, 1, EPI, false>(A, B0, B1, C, M, N, K, lda, ldb, ldc, s, ep);

@@ -1206,6 +1206,34 @@ def test_gemm_bias_gelu_and_residual_epilogues(gpu, M, N, K):
         print(f"gemm bias+residual {M}x{N}x{K} {dt}: bit-equal", flush=True)
 
 
+@pytest.mark.parametrize("M,N,K,bt", [
+    (2047, 2305, 64, True), (2048, 2304, 768, True), (1000, 5000, 1024, True), (8191, 767, 128, True),  # 128x192
+    (500, 11000, 1088, True), (511, 2300, 320, True), (2048, 768, 192, True), (65, 96, 64, True),  # 128x192, 64x96, 64x64
+    (2047, 1000, 1088, True), (2047, 1000, 1088, False), (511, 4096, 64, False)])  # 64x128
+def test_gemm_tile_choices(gpu, M, N, K, bt):
+    """The LDS-DMA kernel's 128x192, 64x96 and 64x128 tiles at their edges, every epilogue: the bits of
+    the register-staged kernel, which the same operands take in rows padded by one element (both sum
+    each output's products in the same order)."""
+    from autokernel_amd.kernels import _ops
+    g = torch.Generator().manual_seed(M + N + K)
+    for dt in (torch.float16, torch.bfloat16):
+        A, B = torch.randn(M, K, generator=g).to(dt).to(gpu), (torch.randn(*((N, K) if bt else (K, N)), generator=g) * 0.1).to(dt).to(gpu)
+        b, r = torch.randn(N, generator=g).to(dt).to(gpu), torch.randn(M, N, generator=g).to(dt).to(gpu)
+        A2, B2 = (torch.nn.functional.pad(t, (0, 1))[:, :-1] for t in (A, B))
+        calls = {"store": lambda c, x, w: _ops.gemm(c, x, w, bt), "bias": lambda c, x, w: _ops.gemm_bias(c, x, w, b, bt),
+                 "gelu": lambda c, x, w: _ops.gemm_bias_gelu(c, x, w, b, bt),
+                 "bias residual": lambda c, x, w: _ops.gemm_bias_residual(c, x, w, b, r, bt),
+                 "residual": lambda c, x, w: _ops.gemm_residual(c, x, w, r, bt)}
+        if N % 128 == 0:
+            cs = torch.randn(2, 100, 32, generator=g).to(gpu)
+            calls["rope"] = lambda c, x, w: _ops.gemm_rope(c, x, w, bt, cs[0], cs[1], 100, 64, N // 2)
+        for name, f in calls.items():
+            got, want = torch.empty_like(r), torch.empty_like(r)
+            f(got, A, B)
+            f(want, A2, B2)
+            assert torch.equal(got, want), (name, M, N, K, bt, dt)
+
+
 @pytest.mark.parametrize("lead,N,K", [((3,), 96, 64), ((2, 5), 72, 40), ((1, 1, 130), 136, 256), ((4, 0), 64, 64),
                                       ((), 33, 24), ((7, 9), 1, 64), ((65,), 80, 1)])
 def test_linear_equals_gemm_forms(gpu, lead, N, K):
