@@ -418,6 +418,52 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
   wait_vmcnt<0>();  // no DMA may still target this block's LDS when its waves end
 }
 
+// Store a block's tile by whole rows through LDS, for a C with rows at odd element offsets (an odd ldc,
+// e.g. a 50257-column vocabulary projection). From the fragments a store instruction writes 64 bytes
+// of each of 16 rows; where those start off a dword they cost twice the requests of dword-aligned
+// ones, while a wave that stores whole rows of the tile pays for a row's two ends only (f16, us, from
+// the fragments / by rows / an even ldc: 2048x50257x768 224 / 199 / 196, 8192x50257x768 838 / 761 / 732;
+// an even ldc is 2 % slower by rows). The tile's halves of BM / 2 rows go to s0 and s1, two of the
+// stages (free once every wave is past the k-loop), 16-byte chunk c of row r at c ^ (r & 7): the 8 lanes
+// of a write (8 rows) or a read (8 chunks) hit distinct bank slots.
+template <typename T, int BM, int BN, int NW, int FM, int FN>
+__device__ __forceinline__ void store_tile_rows(uint16_t* __restrict__ C, int64_t ldc, int M, int N, int m0, int n0,
+                                                int row0, int col0, const f32x4 (&acc)[FM][FN], uint16_t* s0, uint16_t* s1) {
+  constexpr int CPR = BN / 8;  // chunks per row
+  static_assert(BM * CPR % (NW * kWave) == 0 && CPR % 8 == 0, "whole rows of chunks over the block");
+  const int lane = lane_id(), fr = lane & 15, fc = lane >> 4;
+  const auto row = [&](int r) { return (r < BM / 2 ? s0 : s1) + (r % (BM / 2)) * BN; };
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int r = row0 + i * 16 + fr;
+    uint32_t lo[FN], hi[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      lo[j] = (uint32_t)T::from_f(acc[i][j][0]) | ((uint32_t)T::from_f(acc[i][j][1]) << 16);
+      hi[j] = (uint32_t)T::from_f(acc[i][j][2]) | ((uint32_t)T::from_f(acc[i][j][3]) << 16);
+    }
+#pragma unroll
+    for (int j = 0; j + 1 < FN; j += 2) {
+      regroup8(lo[j], lo[j + 1]);
+      regroup8(hi[j], hi[j + 1]);
+      const int c = col0 / 8 + j * 2 + fc;
+      *reinterpret_cast<u32x4*>(row(r) + (c ^ (r & 7)) * 8) = u32x4{lo[j], hi[j], lo[j + 1], hi[j + 1]};
+    }
+    if constexpr (FN % 2 == 1) {
+      const int c = col0 / 8 + (FN - 1) * 2 + fc / 2;
+      *reinterpret_cast<u32x2*>(row(r) + (c ^ (r & 7)) * 8 + (fc & 1) * 4) = u32x2{lo[FN - 1], hi[FN - 1]};
+    }
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int q = threadIdx.x; q < BM * CPR; q += NW * kWave) {
+    const int r = q / CPR, c = q % CPR;
+    const u32x4 o = *reinterpret_cast<const u32x4*>(row(r) + (c ^ (r & 7)) * 8);
+    if (m0 + r < M) store_cols<true, 8>(C + (int64_t)(m0 + r) * ldc + n0 + c * 8, N - n0 - c * 8, o);
+  }
+}
+
 template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int MF, int OCC>
 __global__ __launch_bounds__(WM* WN* kWave, OCC* WM* WN / 4) void gemm_dma(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
@@ -498,6 +544,12 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC* WM* WN / 4) void gemm_dma(
 
   // 16x16 fragment: lane holds C[m0' + lane % 16][n0' + 4 (lane / 16) + 0..3]
   const int fr = lane & 15, fc = lane >> 4;
+  if constexpr (EPI == kEpiStore && NB == 1 && kStage >= BM / 2 * BN && BN % 64 == 0) {
+    if ((ldc & 1) != 0 || ((uintptr_t)C & 3) != 0) {  // uniform over the block
+      store_tile_rows<T, BM, BN, NW, FM, FN>(C, ldc, M, N, m0, n0, wm * WTM, wn * WTN, acc[0], sS0, sS1);
+      return;
+    }
+  }
   tile_epilogue<T, NB, EPI, true, FM, FN>(C, B1, ldc, M, N, m0 + wm * WTM + fr, n0 + wn * WTN + fc * 4, acc, ep);
 }
 

@@ -1209,10 +1209,13 @@ def test_gemm_bias_gelu_and_residual_epilogues(gpu, M, N, K):
 @pytest.mark.parametrize("M,N,K,bt", [
     (2047, 2305, 64, True), (2048, 2304, 768, True), (1000, 5000, 1024, True), (8191, 767, 128, True),  # 128x192
     (500, 11000, 1088, True), (511, 2300, 320, True), (2048, 768, 192, True), (65, 96, 64, True),  # 128x192, 64x96, 64x64
-    (2047, 1000, 1088, True), (2047, 1000, 1088, False), (511, 4096, 64, False)])  # 64x128
+    (2047, 1000, 1088, True), (2047, 1000, 1088, False), (511, 4096, 64, False),  # 64x128
+    # rows at odd offsets: 256x256, 256x192, 128x128, 128x192, 64x128, 64x64
+    (4095, 4095, 1088, True), (2047, 6143, 1088, True), (2047, 2047, 1088, True), (500, 10999, 1088, True),
+    (2047, 999, 1088, True), (511, 767, 64, True)])
 def test_gemm_tile_choices(gpu, M, N, K, bt):
-    """The LDS-DMA kernel's 128x192, 64x96 and 64x128 tiles at their edges, every epilogue: the bits of
-    the register-staged kernel, which the same operands take in rows padded by one element (both sum
+    """The LDS-DMA kernel's 128x192, 64x96 and 64x128 tiles at their edges, every epilogue, and tiles stored
+    by whole rows (rows at odd element offsets): the bits of the register-staged kernel, which the same operands take in rows padded by one element (both sum
     each output's products in the same order)."""
     from autokernel_amd.kernels import _ops
     g = torch.Generator().manual_seed(M + N + K)
