@@ -132,10 +132,11 @@ def require_gpu(op: str, *tensors: torch.Tensor) -> None:
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def stream_of_index(index: int) -> int:
-    if _raw_stream is not None:
-        return _raw_stream(index)
+def _stream_of_index(index: int) -> int:
     return torch.cuda.current_stream(index).cuda_stream
+
+
+stream_of_index = _raw_stream or _stream_of_index
 
 
 def stream_of(t: torch.Tensor) -> int:

@@ -626,7 +626,7 @@ __global__ __launch_bounds__(256) void reduce_cols_short(const typename T::S* __
 // loads take any alignment); the last group is moved back to end at the row's end, so it overlaps
 // its neighbour and both write the same values.
 // Measured on the sum over dim 0 of bf16 [8192, 4096] (67 MB): one thread per output, 16 blocks in
-// all, took 1895 us (35 GB/s).
+// all, took 1895 us (35 GB/s); this takes 14.7 us (4.6 TB/s, both launches).
 constexpr int kColThreads = 256;
 constexpr int kColUnroll = 8;
 
