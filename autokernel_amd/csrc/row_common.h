@@ -137,7 +137,11 @@ struct RowRegs {
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const int idx = gl + j * L;
+      // The zeros are opaque to the compiler: it otherwise loads first and writes constant zeros to the
+      // lanes past the row in an else branch, behind a wait for the load that keeps later loads (the
+      // weights) from overlapping it (layernorm f16 [14223, 448], 56 vectors for 64 lanes: 7.60 us against 7.25).
       u32x4 v = {0u, 0u, 0u, 0u};
+      asm("" : "+v"(v));
       if (idx < sh.nvec) v = ldv<ANY>(row + sh.off(idx));
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e) f[j * T::kVec + e] = T::lane_elem(v, e);
