@@ -238,6 +238,57 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_f32_tile(
   }
   kahan_row(FM - 1);
 
+  // A total that became infinite (an infinite product, an overflow) turns to NaN at the step after it,
+  // inf - inf, where a plain sum stays infinite. So a block that ends with a NaN adds its products again
+  // without compensation and takes those sums for its NaN elements. Finite products pay for the test
+  // (us, without / with: 2048^3 170.6 / 172.2, 4096^3 1334 / 1342), a NaN or infinity anywhere for a second
+  // pass (2048^3 320). Bounding the compensation at every step instead (one v_med3_f32 an element and
+  // 16 of k) costs every product as much as a step of its own: 2048^3 193, 4096^3 1514.
+  bool nan = false;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int f = 0; f < FN; ++f)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) nan |= s[b][i][f][e] != s[b][i][f][e];
+  float* flag = &sA[0][0];  // past the last barrier no wave uses what it reads of the stages
+  if (tid == 0) *flag = 0.f;
+  __syncthreads();
+  if (nan) *flag = 1.f;
+  __syncthreads();
+  if (*flag != 0.f) {  // uniform over the block
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int f = 0; f < FN; ++f) y[b][i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < KT; ++kt) {
+      gload(kt * BK);
+      __syncthreads();
+      sstore(0);
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        load_a(0, h, fa);
+        load_b(0, h, fb);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) mfma_row(i);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int f = 0; f < FN; ++f)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (s[b][i][f][e] != s[b][i][f][e]) s[b][i][f][e] = y[b][i][f][e];
+  }
+
   // Lane group g = lane / 16 holds, of row m, columns 16 f + 4 g + v ([N, K] B) or FN (4 g + v) + f
   // ([K, N] B): either way FN groups of four consecutive columns.
 #pragma unroll

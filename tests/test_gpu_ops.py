@@ -392,6 +392,45 @@ def test_matmul_f32_tiles(gpu, M, N, K, bt):
     assert bool(((out - Ah @ Bh).abs() <= 20 * 2.0 ** -24 * (Ah.abs() @ Bh.abs())).all())
 
 
+def _non_finite_rows(M, K):
+    """A [M, K] of ones whose first rows hold one infinity (at the first, a middle and the last k), opposite
+    infinities, a NaN and finite values whose sum overflows (2e37 a term: 16 terms are finite, 18 are not)."""
+    A = torch.ones(M, K)
+    A[0, 0], A[1, K // 2], A[2, K - 1] = math.inf, -math.inf, math.inf
+    if K > 1:
+        A[3, 0], A[3, K - 1] = math.inf, -math.inf
+    A[4, K // 3] = math.nan
+    A[5] = 2e37
+    return A
+
+
+def _assert_same_non_finite(out, want, what):
+    """Infinities (with their signs) and NaN exactly where want has them."""
+    assert torch.equal(torch.isnan(out), torch.isnan(want)), what
+    assert torch.equal(out.isposinf(), want.isposinf()) and torch.equal(out.isneginf(), want.isneginf()), what
+
+
+@pytest.mark.parametrize("M,N", [(70, 130), (2049, 2100)])
+@pytest.mark.parametrize("K", [1, 8, 16, 17, 32, 40, 48, 64, 1000])
+def test_f32_tiles_keep_infinities(gpu, M, N, K):
+    """fp32 products and gate/up (64 and 128 tiles) with infinities, NaN and overflowing sums at every
+    place in a k-tile give what a plain sum gives: the compensation of an infinite total is bounded,
+    so that the steps after it, those on a tile's zero padding included, leave the total alone."""
+    from autokernel_amd.kernels import _ops, host
+    A = _non_finite_rows(M, K)
+    for bt in (True, False):
+        B = torch.ones(K, N)
+        B[:, 1], B[:, 2] = -1, 0.5
+        Bd = B.t().contiguous().to(gpu).t() if bt else B.to(gpu)
+        out, want = kernels.get("matmul")(A.to(gpu), Bd).cpu(), (A.double() @ B.double()).float()
+        _assert_same_non_finite(out, want, (M, N, K, bt))
+        assert torch.equal(out[6:], want[6:])
+    h = torch.empty(M, N, device=gpu)
+    W = B.t().contiguous().to(gpu)
+    _ops.mlp_gate_up(h, A.to(gpu), W, W, host.ACT_NONE)  # g * u with g = u
+    _assert_same_non_finite(h.cpu(), want * want, (M, N, K, "gate/up"))
+
+
 @pytest.mark.parametrize("M,D,H", [(1, 1, 1), (65, 33, 31), (129, 100, 65), (2048, 64, 1100)])
 @pytest.mark.parametrize("act", ["silu", "relu2"])
 def test_gate_up_f32_tiles(gpu, M, D, H, act):
