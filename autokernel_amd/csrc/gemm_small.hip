@@ -36,6 +36,13 @@ struct SmallVec {
   };
 };
 
+// A compensated sum's correction for the next step. Of a finite total it is at most 2^104 (half a unit in
+// the last place of the largest total, and the rounding of t - s). Once the total is infinite it is
+// NaN or an infinity of the other sign, and the next step would turn the total into NaN; bounded
+// (v_med3_f32 takes a NaN to a finite bound), it leaves an infinite total as it is, as a plain sum does.
+// One VALU operation more per element and 16 of k, hidden behind the loads.
+__device__ __forceinline__ float kahan_bound(float y) { return __builtin_amdgcn_fmed3f(y, -0x1p104f, 0x1p104f); }
+
 // the first `valid` elements of p (16 bytes, or VN columns), zeros after
 template <typename S>
 __device__ __forceinline__ u32x4 small_load_k(const S* p, int valid) {
@@ -195,7 +202,8 @@ __global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typen
               for (int j = 0; j < 4; ++j)
                 y = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(fb[j]), __uint_as_float(x.a[u][i][j]), y, 0, 0, 0);
               const f32x4 t = acc[b][i][c] + y;
-              comp[b][i][c] = y - (t - acc[b][i][c]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) comp[b][i][c][e] = kahan_bound(y[e] - (t[e] - acc[b][i][c][e]));
               acc[b][i][c] = t;
             } else {
               acc[b][i][c] = mfma16x16x32<T>(fb, x.a[u][i], acc[b][i][c]);

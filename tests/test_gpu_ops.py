@@ -431,6 +431,26 @@ def test_f32_tiles_keep_infinities(gpu, M, N, K):
     _assert_same_non_finite(h.cpu(), want * want, (M, N, K, "gate/up"))
 
 
+@pytest.mark.parametrize("M,N", [(7, 100), (16, 5000), (20, 3000), (33, 3000), (40, 5000), (64, 1000)])
+@pytest.mark.parametrize("K", [1, 8, 16, 17, 40, 64, 512, 1100, 4100])
+def test_f32_few_rows_keep_infinities(gpu, M, N, K):
+    """The same at most 64 rows (gemm_small.hip, every configuration): infinities, NaN and overflowing
+    sums in a group's first and last step, with other waves' finite sums and with zero steps behind."""
+    from autokernel_amd.kernels import _ops, host
+    A = _non_finite_rows(M, K)
+    for bt in (True, False):
+        B = torch.ones(K, N)
+        B[:, 1], B[:, 2] = -1, 0.5
+        Bd = B.t().contiguous().to(gpu).t() if bt else B.to(gpu)
+        out, want = kernels.get("matmul")(A.to(gpu), Bd).cpu(), (A.double() @ B.double()).float()
+        _assert_same_non_finite(out, want, (M, N, K, bt))
+        assert torch.equal(out[6:], want[6:])
+    h = torch.empty(M, N, device=gpu)
+    W = B.t().contiguous().to(gpu)
+    _ops.mlp_gate_up(h, A.to(gpu), W, W, host.ACT_NONE)  # g * u with g = u
+    _assert_same_non_finite(h.cpu(), want * want, (M, N, K, "gate/up"))
+
+
 @pytest.mark.parametrize("M,D,H", [(1, 1, 1), (65, 33, 31), (129, 100, 65), (2048, 64, 1100)])
 @pytest.mark.parametrize("act", ["silu", "relu2"])
 def test_gate_up_f32_tiles(gpu, M, D, H, act):
