@@ -279,7 +279,8 @@ __global__ __launch_bounds__(kFrThreads) void fa_rows_merge(const FrArgs a) {
   for (int e = 0; e < VW; ++e) acc[e] = 0.f;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const float f = x + 16 * u >= a.splits || z[u][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(z[u][0] - mb);
+    if (x + 16 * u >= a.splits) continue;  // loaded the last split again: 0 times its infinities would be NaN
+    const float f = z[u][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(z[u][0] - mb);
     l += z[u][1] * f;
 #pragma unroll
     for (int e = 0; e < VW; ++e) acc[e] += v[u][e >> 2][e & 3] * f;

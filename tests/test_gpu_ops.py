@@ -754,6 +754,24 @@ def test_attention_few_rows(gpu, D, dt, B, Hq, Hk, Sq, Sk):
         assert bool(nan[0, :rep].all()) == (1600 * D >= 65520) and not bool(nan[0, rep:].any())
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("Hk,Sk", [(2, 900), (2, 1536), (8, 4096), (1, 4099), (2, 20000)])
+def test_attention_few_rows_keep_infinities(gpu, D, dt, Hk, Sk):
+    """Few query rows per KV head with one infinite value of V in the first, a middle or the last key
+    slice (unsplit, 6, 16, 16 and 64 slices): that dim of the output is that infinity for the head's queries,
+    all of whose weights are 1 / Sk, and every other output stays finite."""
+    Q = torch.zeros(1, 4 * Hk, 1, D, dtype=dt, device=gpu)
+    K, V = (torch.randn(1, Hk, Sk, D, generator=torch.Generator().manual_seed(Sk + D)).to(dt).to(gpu) for _ in range(2))
+    for pos in (0, Sk // 2, Sk - 1):
+        for inf in (math.inf, -math.inf):
+            Vi = V.clone()
+            Vi[0, 0, pos, 3] = inf
+            out = kernels.get("flash_attention")(Q, K, Vi, False)
+            assert bool((out[0, :4, 0, 3] == inf).all()), (pos, inf)
+            assert int(torch.isfinite(out).sum()) == out.numel() - 4, (pos, inf)
+
+
 def test_attention_rectangular_and_scale(gpu):
     g = torch.Generator().manual_seed(6)
     Q = torch.randn(1, 4, 96, 64, generator=g).bfloat16()
