@@ -783,10 +783,11 @@ template <typename T, int NB, int EPI>
 static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C, int64_t M,
                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, bool bt,
                          hipStream_t s, const EpiArgs& ep = EpiArgs{}) {
-  // vec: A and B load as 16-byte k-chunks (C's alignment does not matter: the epilogue checks each
-  // 8-byte store)
+  // vec: A and B load as 16-byte k-chunks. C's alignment does not matter, nor does that of a bias or a
+  // residual (B1 of one product): the epilogue checks each 8-byte access. They must not choose the kernel
+  // either, whose order of the sums an epilogue shares with the plain product.
   bool vec = K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && host_aligned16(A) && host_aligned16(B0) &&
-             (!B1 || EPI == kEpiBias || EPI == kEpiBiasGelu || host_aligned16(B1));
+             (NB == 1 || host_aligned16(B1));
   if (!bt) vec = vec && N % 8 == 0;
   const int m = (int)M, n = (int)N, k = (int)K;
   // LDS-DMA path: K a multiple of 64, 32-bit element offsets

@@ -1314,6 +1314,30 @@ def test_gemm_tile_choices(gpu, M, N, K, bt):
             assert torch.equal(got, want), (name, M, N, K, bt, dt)
 
 
+@pytest.mark.parametrize("M,N,K,bt", [(16, 8192, 4096, True), (64, 4160, 512, False), (64, 4096, 1024, True), (5, 100, 448, True),
+                                      (100, 768, 768, True), (300, 1003, 192, True)])
+def test_epilogue_of_an_unaligned_residual(gpu, M, N, K, bt):
+    """A residual and a bias at any alignment: the epilogues equal the separate product and add bit for
+    bit (the aligned product and the epilogue sum in one order), for shapes on both sides of the few-row
+    rules."""
+    from autokernel_amd.kernels import _ops
+    g = torch.Generator().manual_seed(M + N + K)
+    for dt in (torch.float16, torch.bfloat16):
+        A = torch.randn(M, K, generator=g).to(dt).to(gpu)
+        B = (torch.randn(*((N, K) if bt else (K, N)), generator=g) * 0.1).to(dt).to(gpu)
+        rb, bb = torch.randn(M * N + 7, generator=g).to(dt).to(gpu), torch.randn(N + 7, generator=g).to(dt).to(gpu)
+        plain, biased = torch.empty(M, N, device=gpu, dtype=dt), torch.empty(M, N, device=gpu, dtype=dt)
+        _ops.gemm(plain, A, B, bt)
+        for off in (0, 1, 2, 4, 7):
+            R, b = rb[off:off + M * N].view(M, N), bb[off:off + N]
+            out = torch.empty_like(plain)
+            _ops.gemm_residual(out, A, B, R, bt)
+            assert torch.equal(out, R + plain), ("residual", off, M, N, K, bt, dt)
+            _ops.gemm_bias(biased, A, B, b.clone(), bt)
+            _ops.gemm_bias_residual(out, A, B, b, R, bt)
+            assert torch.equal(out, R + biased), ("bias residual", off, M, N, K, bt, dt)
+
+
 @pytest.mark.parametrize("lead,N,K", [((3,), 96, 64), ((2, 5), 72, 40), ((1, 1, 130), 136, 256), ((4, 0), 64, 64),
                                       ((), 33, 24), ((7, 9), 1, 64), ((65,), 80, 1)])
 def test_linear_equals_gemm_forms(gpu, lead, N, K):
