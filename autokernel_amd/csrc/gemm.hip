@@ -779,6 +779,25 @@ static bool small_rows_win(int64_t M, int64_t N, int64_t K, bool bt, int nb) {
   return N <= 2560 || K >= 2048;
 }
 
+// Shapes and row strides the LDS-DMA path serves (aligned operands provided): K a multiple of 64, 16-byte
+// chunks, 32-bit element offsets.
+static bool dma_shape(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool bt) {
+  return K > 0 && K % kBK == 0 && lda % 8 == 0 && ldb % 8 == 0 && (bt || N % 8 == 0) && M * lda < INT_MAX &&
+         (bt ? N : K) * ldb < INT_MAX;
+}
+
+// The period of a batch's kernel choice. A product of at most kSmallM rows that small_rows_win leaves to
+// the LDS-DMA kernel takes gemm_small where its operands are off 16 bytes, and the two sum in different
+// orders. Every item of a batch has to equal its 2-D product, so where the batch strides move items on
+// and off 16 bytes, items z, z + p, ... are one launch.
+static int64_t batch_period(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t stride_a,
+                            int64_t stride_b, bool bt) {
+  if (M > kSmallM || !dma_shape(M, N, K, lda, ldb, bt) || small_rows_win(M, N, K, bt, 1)) return 1;
+  int64_t p = 1;
+  while ((p * stride_a) % 8 != 0 || (p * stride_b) % 8 != 0) p *= 2;
+  return p;
+}
+
 template <typename T, int NB, int EPI>
 static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C, int64_t M,
                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, bool bt,
@@ -786,15 +805,11 @@ static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C,
   // vec: A and B load as 16-byte k-chunks. C's alignment does not matter, nor does that of a bias or a
   // residual (B1 of one product): the epilogue checks each 8-byte access. They must not choose the kernel
   // either, whose order of the sums an epilogue shares with the plain product.
-  bool vec = K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && host_aligned16(A) && host_aligned16(B0) &&
+  bool vec = K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && (bt || N % 8 == 0) && host_aligned16(A) && host_aligned16(B0) &&
              (NB == 1 || host_aligned16(B1));
-  if (!bt) vec = vec && N % 8 == 0;
   const int m = (int)M, n = (int)N, k = (int)K;
-  // LDS-DMA path: K a multiple of 64, 32-bit element offsets
-  const bool dma = vec && K % kBK == 0 && K > 0 && (bt || N >= 8) && M * lda < INT_MAX &&
-                   (bt ? N : K) * ldb < INT_MAX;
-  // Few rows: always for operands that path cannot read, by shape for those it can. The batch (its
-  // strides included) has no say, so that every item of a batched product equals the 2-D product.
+  const bool dma = vec && dma_shape(M, N, K, lda, ldb, bt);
+  // Few rows: always for operands that path cannot read, by shape for those it can.
   if (M <= kSmallM && K > 0 && (bt || NB == 1) && (!dma || small_rows_win(M, N, K, bt, NB)))
     return launch_gemm_small<T, NB, EPI>(A, B0, B1, C, M, N, K, lda, ldb, ldc, bt, s, ep);
   vec = vec && ep.batch_a % 8 == 0 && ep.batch_b % 8 == 0;
@@ -933,27 +948,32 @@ extern "C" int ak_gemm_batched(int dtype, const void* A, const void* B, void* C,
   if (cdiv(M, 128) * cdiv(N, 128) > INT_MAX) return AK_EINVAL;
   const bool bt = b_trans != 0;
   const int esz = dtype == AK_F32 ? 4 : 2;
+  const int64_t period = dtype == AK_F32 ? 1 : batch_period(M, N, K, lda, ldb, stride_a, stride_b, bt);
+  const int64_t sa = stride_a * period, sb = stride_b * period, sc = stride_c * period;
   // grid z holds at most 65535 items: larger batches run in chunks
   constexpr int64_t kMaxZ = 65535;
-  for (int64_t z0 = 0; z0 < batch; z0 += kMaxZ) {
-    const int64_t nz = batch - z0 < kMaxZ ? batch - z0 : kMaxZ;
-    const char* a = (const char*)A + z0 * stride_a * esz;
-    const char* b = (const char*)B + z0 * stride_b * esz;
-    char* c = (char*)C + z0 * stride_c * esz;
-    int st = AK_OK;
-    if (dtype == AK_F32) {
-      st = launch_gemm32(a, b, c, M, N, K, lda, ldb, ldc, bt, stream, (int)nz, stride_a, stride_b, stride_c);
-    } else {
-      EpiArgs ep;
-      ep.batch = (int)nz;
-      ep.batch_a = stride_a;
-      ep.batch_b = stride_b;
-      ep.batch_c = stride_c;
-      if (dtype == AK_F16) st = launch_gemm16<TF16, 1, kEpiStore>(a, b, nullptr, c, M, N, K, lda, ldb, ldc, bt, stream, ep);
-      else if (dtype == AK_BF16) st = launch_gemm16<TBF16, 1, kEpiStore>(a, b, nullptr, c, M, N, K, lda, ldb, ldc, bt, stream, ep);
-      else return AK_EINVAL;
+  for (int64_t r = 0; r < period && r < batch; ++r) {
+    const int64_t items = cdiv(batch - r, period);
+    for (int64_t z0 = 0; z0 < items; z0 += kMaxZ) {
+      const int64_t nz = items - z0 < kMaxZ ? items - z0 : kMaxZ, first = r + z0 * period;
+      const char* a = (const char*)A + first * stride_a * esz;
+      const char* b = (const char*)B + first * stride_b * esz;
+      char* c = (char*)C + first * stride_c * esz;
+      int st = AK_OK;
+      if (dtype == AK_F32) {
+        st = launch_gemm32(a, b, c, M, N, K, lda, ldb, ldc, bt, stream, (int)nz, sa, sb, sc);
+      } else {
+        EpiArgs ep;
+        ep.batch = (int)nz;
+        ep.batch_a = sa;
+        ep.batch_b = sb;
+        ep.batch_c = sc;
+        if (dtype == AK_F16) st = launch_gemm16<TF16, 1, kEpiStore>(a, b, nullptr, c, M, N, K, lda, ldb, ldc, bt, stream, ep);
+        else if (dtype == AK_BF16) st = launch_gemm16<TBF16, 1, kEpiStore>(a, b, nullptr, c, M, N, K, lda, ldb, ldc, bt, stream, ep);
+        else return AK_EINVAL;
+      }
+      if (st != AK_OK) return st;
     }
-    if (st != AK_OK) return st;
   }
   return AK_OK;
 }

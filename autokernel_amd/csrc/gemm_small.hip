@@ -18,8 +18,10 @@
 // Measured (us, before / now; three rotating operand sets): bf16 nt 1 x 4096 x 4096 13.9 / 9.4, 16 x 4096 x
 // 11008 30 / 26, nn 29 x 3702 x 10112 (repacked before) 237 / 64, nn 10 x 1536 x 246 28 / 12; gate/up
 // 16 x 4096 -> 11008 65 / 55; f32 nt 16 x 11008 x 4096 563 / 57, nn 28 x 553 x 6656 940 / 53.
-// WV and U, which fix the order of the sums, depend on M, N and K only: a batched product equals its
-// items, and an epilogue equals the separate op, bit for bit.
+// WV and U, which fix the order of the sums, depend on M, N, K, B's layout and NB only, so that a batched
+// product equals its items, and an epilogue equals the separate op, bit for bit. Which products come here
+// also depends on the alignment of A and B (launch_gemm16), which a product and its epilogue forms share;
+// ak_gemm_batched launches items of different alignment apart (batch_period).
 #include <limits.h>
 
 #include "gemm_common.h"

@@ -351,6 +351,25 @@ def test_matmul_few_rows(gpu, M, N, K, dt):
     assert torch.equal(kernels.get("matmul")(batch, torch.stack([Bt, Bt]).transpose(1, 2))[1], _gemm(Ad, Bt.t()))
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 128, 448), (64, 4160, 1024), (33, 2048, 512), (5, 136, 64), (16, 768, 768), (3, 100, 70)])
+@pytest.mark.parametrize("pad_a,pad_b", [(1, 3), (2, 0), (4, 8), (0, 1), (8, 6)])
+def test_batched_few_rows_of_any_stride(gpu, M, N, K, pad_a, pad_b):
+    """Items of at most 64 rows whose batch strides put them on and off 16 bytes, more items than the
+    period of eight: each equals its 2-D product bit for bit, on both sides of the few-row rules and for
+    an operand shared by the batch."""
+    from autokernel_amd.kernels import host
+    g = torch.Generator().manual_seed(M + N + K + pad_a + 10 * pad_b)
+    Z = 11
+    for dt in (torch.float16, torch.bfloat16):
+        A = torch.randn(Z * (M * K + pad_a), generator=g).to(dt).to(gpu).as_strided((Z, M, K), (M * K + pad_a, K, 1))
+        Bf = torch.randn(Z * (K * N + pad_b), generator=g).to(dt).to(gpu)
+        for B in (Bf.as_strided((Z, N, K), (K * N + pad_b, K, 1)).transpose(1, 2),
+                  Bf.as_strided((Z, K, N), (K * N + pad_b, N, 1)), Bf.as_strided((Z, K, N), (0, N, 1))):
+            out = kernels.get("matmul")(A, B)
+            for z in range(Z):
+                assert torch.equal(out[z], host._gemm(A[z], B[z])), (z, M, N, K, pad_a, pad_b, dt)
+
+
 @pytest.mark.parametrize("M,D,H", [(1, 513, 77), (16, 512, 4097), (17, 600, 5000), (33, 1000, 4096), (64, 31, 33), (64, 700, 5000)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
 @pytest.mark.parametrize("act", ["silu", "gelu", "relu2", "none"])
