@@ -213,6 +213,8 @@ inline void launch_timed(F kernel, dim3 grid, dim3 block, uint32_t shmem, hipStr
 
 inline bool host_aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// Whether a one-dimensional grid can be launched: HIP refuses 2^32 work-items and more.
+inline bool grid_fits(int64_t blocks, int threads) { return blocks < ((int64_t)1 << 32) / threads; }
 
 // floor(n / d) for n, d < 2^31 as one multiply and one shift (Granlund and Montgomery, "Division
 // by invariant integers using multiplication", 1994): with s = ceil(log2 d) and

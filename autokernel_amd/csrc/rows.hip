@@ -775,7 +775,9 @@ static int launch_reduce(const void* x, void* y, int64_t outer, int64_t red_n, i
     return record_launch();
   }
   ColPlan p = plan_cols(outer, red_n, inner, T::kVec);
-  if (p.short_rows || p.col_blocks * outer > INT_MAX) {
+  // (a block of the column kernel takes two to four threads per output, or more where inner is narrow, so
+  // one thread per output still fits where its grid does not)
+  if (p.short_rows || !grid_fits(p.col_blocks * outer, kColThreads)) {
     reduce_cols_short<T, MAX><<<(unsigned)cdiv(outer * inner, 256), 256, 0, s>>>(xp, yp, outer, red_n, inner);
     return record_launch();
   }

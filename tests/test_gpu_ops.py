@@ -865,6 +865,17 @@ def test_reduce_strided_dim(gpu, shape, dim, dt):
     assert torch.equal(torch.isnan(m), torch.isnan(xn.max(dim).values))
 
 
+def test_reduce_strided_dim_of_many_outputs(gpu):
+    """A reduction whose column blocks would pass the 2^32 work-items of a grid (2^24 blocks of 256, here
+    for 2^31 outputs of one row each) runs one thread per output."""
+    if torch.cuda.mem_get_info()[0] < 12 << 30:
+        pytest.skip("needs 9 GB")
+    x = torch.zeros(1 << 19, 1, 4096, dtype=torch.float16, device=gpu)
+    x[0, 0, 0], x[-1, 0, -1], x[1234, 0, 77] = 1, 2, 3
+    y = kernels.get("reduce")(x, 1)
+    assert y.shape == (1 << 19, 4096) and torch.equal(y, x[:, 0])
+
+
 def test_softmax_dim_and_layernorm_none(gpu):
     g = torch.Generator().manual_seed(8)
     x = torch.randn(33, 17, 5, generator=g)
