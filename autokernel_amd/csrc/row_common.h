@@ -195,12 +195,16 @@ inline bool plan_row(int64_t nvec, int kvec, RowPlan* p, int want = 4) {
   return true;
 }
 
-// The plan for a row of `cols` elements; any: at any alignment (the most vectors it may cover, or, where
-// those do not fit, as many as it needs).
-inline bool plan_row_cols(int64_t cols, int kvec, bool any, RowPlan* p, int want = 4) {
+// The plan for `rows` rows of `cols` elements; any: at any alignment (the most vectors a row may cover, or,
+// where those do not fit, as many as it needs). None where the rows' lanes pass a grid's work-items (2^22
+// rows of 1024 lanes); the kernels of 256 threads per row take four times as many.
+inline bool plan_row_cols(int64_t rows, int64_t cols, int kvec, bool any, RowPlan* p, int want = 4) {
   if (cols < kvec) return false;
-  if (!any) return plan_row(cols / kvec, kvec, p, want);
-  return plan_row(cdiv(cols + kvec - 1, kvec), kvec, p, want) || plan_row(cdiv(cols, kvec), kvec, p, want);
+  const bool fits = !any ? plan_row(cols / kvec, kvec, p, want)
+                         : plan_row(cdiv(cols + kvec - 1, kvec), kvec, p, want) || plan_row(cdiv(cols, kvec), kvec, p, want);
+  if (!fits) return false;
+  const int threads = p->L < 256 ? 256 : p->L;  // per block (RowGeom)
+  return grid_fits(cdiv(rows, threads / p->L), threads);
 }
 
 }  // namespace ak

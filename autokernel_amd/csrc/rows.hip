@@ -106,7 +106,7 @@ static int launch_rmsnorm(const void* x, const void* w, void* y, int64_t rows, i
   RowPlan plan;
   const bool any = cols % T::kVec != 0 || !host_aligned16(x) || !host_aligned16(y) || !host_aligned16(w);
   bool handled = false;
-  if (plan_row_cols(cols, T::kVec, any, &plan)) {
+  if (plan_row_cols(rows, cols, T::kVec, any, &plan)) {
     AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
       rmsnorm_rows<T, L, VPT, FORM, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, wp, yp, rows, (int)cols, eps);
@@ -224,7 +224,7 @@ static int launch_layernorm(const void* x, const void* w, const void* b, void* y
   const bool any = cols % T::kVec != 0 || !host_aligned16(x) || !host_aligned16(y) ||
                    (w && !host_aligned16(w)) || (b && !host_aligned16(b));
   bool handled = false;
-  if (plan_row_cols(cols, T::kVec, any, &plan)) {
+  if (plan_row_cols(rows, cols, T::kVec, any, &plan)) {
     AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
       layernorm_rows<T, L, VPT, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, wp, bp, yp, rows, (int)cols, eps);
@@ -401,7 +401,7 @@ static int launch_softmax(const void* x, void* y, int64_t rows, int64_t cols, hi
   // RoPE(q), RoPE(k), softmax step.
   const int nt_out = rows * cols * (int64_t)sizeof(S) > ((int64_t)256 << 20);
   const bool any = cols % T::kVec != 0 || !host_aligned16(x) || !host_aligned16(y);
-  if (plan_row_cols(cols, T::kVec, any, &plan)) {
+  if (plan_row_cols(rows, cols, T::kVec, any, &plan)) {
     AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
       launch_timed(softmax_rows<T, L, VPT, ANY>, grid, dim3(RowGeom<L>::kThreads), 0, s, xp, yp, rows, (int)cols, nt_out);
@@ -539,7 +539,7 @@ static int launch_ce(const void* logits, const int64_t* tgt, float* loss, void* 
   RowPlan plan;
   const bool any = vocab % T::kVec != 0 || !host_aligned16(logits);
   bool handled = rows == 0;  // no rows: only the mean kernel runs (0 / 0 = NaN, as torch gives)
-  const bool planned = plan_row_cols(vocab, T::kVec, any, &plan);
+  const bool planned = plan_row_cols(rows, vocab, T::kVec, any, &plan);
   // 16-bit rows past 32768 columns, and unaligned ones past 16384, stream once the rows fill the chip: a
   // register-cached block of theirs leaves room for one row per CU (us, ce_rows / ce_stream, f16: 4096 x
   // 50264 98 / 81, 4096 x 32769 78 / 56, 4096 x 16385 36 / 30; but 100 x 65536 9.0 / 12.4, aligned 4096 x
@@ -765,7 +765,7 @@ static int launch_reduce(const void* x, void* y, int64_t outer, int64_t red_n, i
     RowPlan plan;
     const bool any = cols % T::kVec != 0 || !host_aligned16(x);
     bool handled = false;
-    if (plan_row_cols(cols, T::kVec, any, &plan, 2)) {
+    if (plan_row_cols(rows, cols, T::kVec, any, &plan, 2)) {
       AK_ANY_SWITCH(any, AK_ROW_SWITCH({
         const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
         reduce_rows<T, L, VPT, MAX, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, yp, rows, (int)cols);

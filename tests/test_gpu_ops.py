@@ -876,6 +876,17 @@ def test_reduce_strided_dim_of_many_outputs(gpu):
     assert y.shape == (1 << 19, 4096) and torch.equal(y, x[:, 0])
 
 
+def test_row_ops_of_many_rows(gpu):
+    """2^22 rows of a width that takes 1024 lanes (8193 f16 values for a sum) would pass the 2^32
+    work-items of a grid: such rows run the looped kernel of 256 threads per row."""
+    if torch.cuda.mem_get_info()[0] < 90 << 30:
+        pytest.skip("needs 69 GB")
+    x = torch.zeros(1 << 22, 8193, dtype=torch.float16, device=gpu)
+    x[0, 0], x[-1, -1], x[1234, 4000:4003] = 1, 2, 3
+    y = kernels.get("reduce")(x, -1)
+    assert y[0] == 1 and y[-1] == 2 and y[1234] == 9 and int((y != 0).sum()) == 3
+
+
 def test_softmax_dim_and_layernorm_none(gpu):
     g = torch.Generator().manual_seed(8)
     x = torch.randn(33, 17, 5, generator=g)
