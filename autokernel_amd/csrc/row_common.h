@@ -19,6 +19,8 @@
 // [4096, 20001] 92 -> 62, [16000, 1235] 37 -> 15; cross-entropy fp32 [4096, 20001] 144 -> 58. Widths just
 // under 65536, whose rows take straddling vectors, are level (softmax [1024, 65535] 62 -> 66).
 #pragma once
+#include <limits.h>
+
 #include "ak_common.h"
 
 namespace ak {
@@ -94,12 +96,15 @@ template <typename T, bool ANY>
 struct RowShape {
   int cols, nvec, skew;  // skew: elements between the aligned address at or before the row and its start
   // most: vectors the row's lanes hold. A row that an end piece would take past it (a width just under
-  // the widest one) takes its vectors from its own start instead.
-  __device__ __forceinline__ RowShape(const typename T::S* row, int cols_, bool active, int most = 1 << 30)
+  // the widest one, or under 2^31) takes its vectors from its own start instead.
+  __device__ __forceinline__ RowShape(const typename T::S* row, int cols_, bool active, int most = INT_MAX / T::kVec)
       : cols(cols_) {
     skew = ANY ? (int)(((uintptr_t)row & 15u) / sizeof(typename T::S)) : 0;
-    if (ANY && (cols + skew + T::kVec - 1) / T::kVec > most) skew = 0;
-    nvec = !active ? 0 : ANY ? (cols + skew + T::kVec - 1) / T::kVec : cols / T::kVec;
+    if (ANY && count() > most) skew = 0;
+    nvec = !active ? 0 : ANY ? count() : cols / T::kVec;
+  }
+  __device__ __forceinline__ int count() const {
+    return (int)(((unsigned)cols + (unsigned)skew + T::kVec - 1) / T::kVec);
   }
   __device__ __forceinline__ int off(int idx) const {
     return ANY ? min(max(idx * T::kVec - skew, 0), cols - T::kVec) : idx * T::kVec;
@@ -108,7 +113,7 @@ struct RowShape {
   template <typename F>
   __device__ __forceinline__ void each(int idx, const float* v, F fn) const {
     const int first = idx * T::kVec - skew;
-    if (!ANY || (first >= 0 && first + T::kVec <= cols)) {
+    if (!ANY || (first >= 0 && first <= cols - T::kVec)) {
 #pragma unroll
       for (int e = 0; e < T::kVec; ++e) fn(v[e]);
     } else {

@@ -876,6 +876,24 @@ def test_reduce_strided_dim_of_many_outputs(gpu):
     assert y.shape == (1 << 19, 4096) and torch.equal(y, x[:, 0])
 
 
+def test_softmax_cross_entropy_of_the_widest_row(gpu):
+    """One row of 2^31 - 1 bf16 values, whose vector count rounds past an int, from an aligned address and
+    seven elements past one: equal values give log(2^31 - 1) and 2^-31 everywhere."""
+    from autokernel_amd.kernels import _ops
+    if torch.cuda.mem_get_info()[0] < 12 << 30:
+        pytest.skip("needs 9 GB")
+    n = 2 ** 31 - 1
+    buf = torch.zeros(n + 7, dtype=torch.bfloat16, device=gpu)
+    out, loss = torch.empty((), device=gpu, dtype=torch.bfloat16), torch.empty(1, device=gpu)
+    for off in (0, 7):
+        x = buf[off:off + n].view(1, n)
+        _ops.cross_entropy(out, loss, x, torch.tensor([n - 1], device=gpu), -100)
+        assert abs(float(loss) - math.log(n)) <= 0.06, (off, float(loss))  # rounded to bf16: 2^-4 at 21
+        y = kernels.get("softmax")(x)
+        assert bool((y == 2.0 ** -31).all()), off
+        del y
+
+
 def test_row_ops_of_many_rows(gpu):
     """2^22 rows of a width that takes 1024 lanes (8193 f16 values for a sum) would pass the 2^32
     work-items of a grid: such rows run the looped kernel of 256 threads per row."""
