@@ -340,7 +340,8 @@ __device__ __forceinline__ void stream_ms(const typename T::S* xr, int cols, flo
 }
 
 // Streaming softmax: the online pass above, then a second read of the row (from the caches when they
-// still hold it) that writes exp2((x - M) log2 e) / S.
+// still hold it) that writes exp2((x - M) log2 e) / S. The write pass takes the row's whole aligned vectors
+// and the few elements at its ends one by one, so that no lane reads what another writes: y may be x.
 template <typename T>
 __global__ __launch_bounds__(kLoopThreads) void softmax_stream(const typename T::S* __restrict__ x,
                                                                typename T::S* __restrict__ y, int cols) {
@@ -350,21 +351,29 @@ __global__ __launch_bounds__(kLoopThreads) void softmax_stream(const typename T:
   float M, S;
   stream_ms<T>(xr, cols, red, &M, &S);
   const float inv = 1.0f / S;
-  const RowShape<T, true> sh(xr, cols, true);
-  for (int b = threadIdx.x; b < sh.nvec; b += kLoopThreads * kStreamUnroll) {
+  auto value = [&](float v) { return fast_exp2((v - M) * kLog2e) * inv; };
+  const int skew = RowShape<T, true>(xr, cols, true).skew, head = skew ? T::kVec - skew : 0;
+  const int nvec = (cols - head) / T::kVec, tail = head + nvec * T::kVec;
+  const typename T::S* xv = xr + head;
+  typename T::S* yv = yr + head;
+  for (int b = threadIdx.x; b < nvec; b += kLoopThreads * kStreamUnroll) {
     u32x4 p[kStreamUnroll];
 #pragma unroll
     for (int u = 0; u < kStreamUnroll; ++u)
-      p[u] = ldv<true>(xr + sh.off(min(b + u * kLoopThreads, sh.nvec - 1)));
+      p[u] = ldv<true>(xv + min(b + u * kLoopThreads, nvec - 1) * T::kVec);
 #pragma unroll
     for (int u = 0; u < kStreamUnroll; ++u)
-      if (b + u * kLoopThreads < sh.nvec) {
+      if (b + u * kLoopThreads < nvec) {
         u32x4 o;
 #pragma unroll
-        for (int e = 0; e < T::kVec; ++e) T::set_elem(o, e, fast_exp2((T::lane_elem(p[u], e) - M) * kLog2e) * inv);
-        stv<true>(yr + sh.off(b + u * kLoopThreads), o);
+        for (int e = 0; e < T::kVec; ++e) T::set_elem(o, e, value(T::lane_elem(p[u], e)));
+        stv<true>(yv + (b + u * kLoopThreads) * T::kVec, o);
       }
   }
+  // one lane per element: the first ones take the head, the next ones the tail (fewer than kVec each)
+  const int t = threadIdx.x, past = t - head;
+  if (t < head) yr[t] = T::from_f(value(T::to_f(xr[t])));
+  else if (past < cols - tail) yr[tail + past] = T::from_f(value(T::to_f(xr[tail + past])));
 }
 
 template <typename T>

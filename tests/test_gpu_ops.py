@@ -894,6 +894,22 @@ def test_softmax_cross_entropy_of_the_widest_row(gpu):
         del y
 
 
+@pytest.mark.parametrize("cols", [3, 9, 1000, 4097, 32769, 65535, 65544, 70001, 131075])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+def test_softmax_in_place(gpu, cols, dt):
+    """y may be x: the same bits as into another buffer, at two alignments, for cached and streamed rows."""
+    from autokernel_amd.kernels import _ops
+    rows = 40
+    buf = torch.randn(rows * cols + 8, generator=torch.Generator().manual_seed(cols)).to(dt).to(gpu)
+    for off in (0, 3):
+        x = buf[off:off + rows * cols].view(rows, cols)
+        y = torch.empty_like(buf)[off:off + rows * cols].view(rows, cols)
+        _ops.softmax(y, x)
+        z = buf.clone()[off:off + rows * cols].view(rows, cols)
+        _ops.softmax(z, z)
+        assert torch.equal(z, y), (cols, dt, off)
+
+
 def test_row_ops_of_many_rows(gpu):
     """2^22 rows of a width that takes 1024 lanes (8193 f16 values for a sum) would pass the 2^32
     work-items of a grid: such rows run the looped kernel of 256 threads per row."""
