@@ -146,6 +146,15 @@ __global__ __launch_bounds__(kFrThreads, 2) void fa_rows(const FrArgs a) {
     for (int x = 0; x < NS; ++x)
 #pragma unroll
       for (int t = 0; t < 2; ++t) s[t] = mfma16x16x32<T>(st.k[t][x], qf[x], s[t]);
+    if constexpr (T::kCode == AK_F16) {
+      // f16 scores round to -inf past the range and weigh nothing, however small the scale. (One at the
+      // other end makes its row NaN, see fr_store_row.)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (s[t][v] <= -a.thr) s[t][v] = -INFINITY;
+    }
     if (k0 + kFrKeys > kend) {
       const int left = kend - (k0 + 8 * g);
 #pragma unroll

@@ -791,6 +791,31 @@ def test_attention_few_rows_keep_infinities(gpu, D, dt, Hk, Sk):
             assert int(torch.isfinite(out).sum()) == out.numel() - 4, (pos, inf)
 
 
+@pytest.mark.parametrize("layout", ["dense", "shared keys", "wide rows"])
+@pytest.mark.parametrize("Sk", [64, 4096])
+def test_attention_few_rows_f16_scores_below_range(gpu, Sk, layout):
+    """f16 scores below the range (-81920) beside ordinary ones, at a scale small enough that their
+    distance alone would not hide them: the reference's f16 scores are -inf there, so those keys weigh
+    nothing, for dense keys, keys of stride 0 and rows whose bytes pass 2^31."""
+    D = 64
+    K = torch.zeros(1, 2, Sk, D)
+    K[:, :, ::2] = -40.0
+    Q, V = torch.full((1, 4, 1, D), 32.0), torch.randn(1, 2, Sk, D, generator=torch.Generator().manual_seed(Sk))
+    if layout == "shared keys":  # every key the same: all of them below the range, a row of NaN
+        Kd = torch.full((1, 2, 1, D), -40.0, dtype=torch.float16, device=gpu).expand(1, 2, Sk, D)
+    else:
+        stride = 1 << 19 if layout == "wide rows" and Sk == 4096 else D
+        buf = torch.empty((Sk - 1) * stride + 2 * D, dtype=torch.float16, device=gpu)
+        Kd = buf.as_strided((1, 2, Sk, D), (0, D, stride, 1)) if stride > D else torch.empty(1, 2, Sk, D, dtype=torch.float16, device=gpu)
+        Kd.copy_(K)
+    out = fa_mod.attention(Q.half().to(gpu), Kd, V.half().to(gpu), False, 1e-5).double().cpu()
+    if layout == "shared keys":
+        assert bool(torch.isnan(out).all())
+        return
+    want = V.half().double()[:, :, 1::2].mean(2, keepdim=True).repeat_interleave(2, 1)
+    assert float((out - want).abs().max()) <= (2 * 2.0 ** -11 + Sk * 2.0 ** -22) * float(V.abs().max())
+
+
 def test_attention_rectangular_and_scale(gpu):
     g = torch.Generator().manual_seed(6)
     Q = torch.randn(1, 4, 96, 64, generator=g).bfloat16()
