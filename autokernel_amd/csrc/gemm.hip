@@ -810,7 +810,7 @@ static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C,
   const int m = (int)M, n = (int)N, k = (int)K;
   const bool dma = vec && dma_shape(M, N, K, lda, ldb, bt);
   // Few rows: always for operands that path cannot read, by shape for those it can.
-  if (M <= kSmallM && K > 0 && (bt || NB == 1) && (!dma || small_rows_win(M, N, K, bt, NB)))
+  if (M <= kSmallM && N <= small_max_n(NB) && K > 0 && (bt || NB == 1) && (!dma || small_rows_win(M, N, K, bt, NB)))
     return launch_gemm_small<T, NB, EPI>(A, B0, B1, C, M, N, K, lda, ldb, ldc, bt, s, ep);
   vec = vec && ep.batch_a % 8 == 0 && ep.batch_b % 8 == 0;
   if (bt && dma && vec) {

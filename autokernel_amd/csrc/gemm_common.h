@@ -294,8 +294,10 @@ __device__ __forceinline__ void tile_epilogue(uint16_t* __restrict__ C, const ui
   }
 }
 
-// Products with at most kSmallM rows of A (gemm_small.hip); any alignment, any K > 0.
+// Products with at most kSmallM rows of A (gemm_small.hip); any alignment, any K > 0. N stays below the
+// 2^32 work-items of a grid: at most 16 per column (32 for gate/up).
 constexpr int64_t kSmallM = 64;
+constexpr int64_t small_max_n(int nb) { return ((int64_t)1 << 28) / nb - 64; }
 template <typename T, int NB, int EPI>
 int launch_gemm_small(const void* A, const void* B0, const void* B1, void* C, int64_t M, int64_t N, int64_t K,
                       int64_t lda, int64_t ldb, int64_t ldc, bool bt, hipStream_t s, const EpiArgs& ep);

@@ -338,8 +338,8 @@ static bool small_tile32(int64_t M, int64_t N, int64_t batch, int bn_big) {
 // (16) rows, whose tiles fill the chip (us, tiles / gemm_small: 48 x 50257 x 768 84 / 108, 33 x 14976 x 179
 // 10.8 / 15.1, gate/up 64 x 5120 -> 13824 264 / 317; but 64 x 11008 x 4096 142 / 123, 64 x 4096 x 4096
 // 142 / 38).
-static bool small_rows32(int64_t M, int64_t N, int64_t K) {
-  if (M > kSmallM || K == 0) return false;
+static bool small_rows32(int64_t M, int64_t N, int64_t K, int nb) {
+  if (M > kSmallM || K == 0 || N > small_max_n(nb)) return false;
   if (M > 32 && N > 4096 && (N > 12288 || K < 1024)) return false;
   return !(M > 16 && N > 8192 && K < 512);
 }
@@ -357,7 +357,7 @@ static void launch_tile32(const void* A, const void* B0, const void* B1, void* C
 int launch_gemm32(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                   int64_t ldb, int64_t ldc, bool bt, hipStream_t s, int batch, int64_t batch_a, int64_t batch_b,
                   int64_t batch_c) {
-  if (small_rows32(M, N, K)) {
+  if (small_rows32(M, N, K, 1)) {
     EpiArgs ep;
     ep.batch = batch;
     ep.batch_a = batch_a;
@@ -380,7 +380,7 @@ int launch_gemm32(const void* A, const void* B, void* C, int64_t M, int64_t N, i
 
 int launch_gate_up32(const void* x, const void* wg, const void* wu, void* h, int64_t M, int64_t H, int64_t D,
                      int epi, hipStream_t s) {
-  if (small_rows32(M, H, D)) {
+  if (small_rows32(M, H, D, 2)) {
     const EpiArgs ep;
     switch (epi) {
       case kEpiSilu: return launch_gemm_small<TF32, 2, kEpiSilu>(x, wg, wu, h, M, H, D, D, D, H, true, s, ep);

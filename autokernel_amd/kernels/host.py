@@ -199,9 +199,11 @@ def reduce_max(x: torch.Tensor, dim: int = -1) -> torch.Tensor:
 # 28 us repacked; 4095^3: 882 against 228 us). Above this size they are copied once into zero-padded
 # operands whose K is a multiple of 64. The extra products are exact zeros at the end of each sum,
 # so the result is the same.
-# Products of at most _SMALL_M rows read any alignment in place (gemm_small.hip) and are not repacked.
+# Products of at most _SMALL_M rows and _SMALL_MAX_N columns read any alignment in place (gemm_small.hip)
+# and are not repacked.
 _REPACK_MIN_MNK = 1 << 21
 _SMALL_M = 64
+_SMALL_MAX_N = (1 << 28) - 64
 
 
 def _ld(t: torch.Tensor) -> int:
@@ -241,7 +243,7 @@ def _gemm(A: torch.Tensor, B: torch.Tensor, out: torch.Tensor | None = None, spl
     C = out if out is not None else torch.empty((M, N), device=A.device, dtype=A.dtype)
     if K == 0:
         return C.zero_()
-    if A.dtype != torch.float32 and M > _SMALL_M and M * N * K >= _REPACK_MIN_MNK and not (
+    if A.dtype != torch.float32 and (M > _SMALL_M or N > _SMALL_MAX_N) and M * N * K >= _REPACK_MIN_MNK and not (
             K % 8 == 0 and _ld(A) % 8 == 0 and _ld(Bs) % 8 == 0 and A.data_ptr() % 16 == 0
             and Bs.data_ptr() % 16 == 0 and (bt or N % 8 == 0)):
         A, Bs, bt, K = _repack(A, Bs, bt, N, K)

@@ -370,6 +370,24 @@ def test_batched_few_rows_of_any_stride(gpu, M, N, K, pad_a, pad_b):
                 assert torch.equal(out[z], host._gemm(A[z], B[z])), (z, M, N, K, pad_a, pad_b, dt)
 
 
+@pytest.mark.parametrize("dt,K", [(torch.float16, 8), (torch.float16, 7), (torch.float32, 4)], ids=["f16", "f16 odd", "f32"])
+def test_matmul_few_rows_of_many_columns(gpu, dt, K):
+    """2^28 columns against one row: gemm_small's 16 work-items per column would pass a grid's 2^32, so
+    such products stay on the tile kernels; gate/up the same at 2^27."""
+    from autokernel_amd.kernels import _ops, host
+    n = 1 << 28
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 40 GB (rows of odd length are repacked to 64 values)")
+    W = torch.zeros(n, K, dtype=dt, device=gpu)
+    W[:, 0], W[-1], W[n // 2 + 1, 1] = 1, 3, 2
+    x = torch.ones(1, K, dtype=dt, device=gpu)
+    y = kernels.get("matmul")(x, W.t())[0]
+    assert y[0] == 1 and y[-1] == 3 * K and y[n // 2 + 1] == 3 and int((y == 1).sum()) == n - 2
+    h = torch.empty(1, n // 2, dtype=dt, device=gpu)
+    _ops.mlp_gate_up(h, x, W[:n // 2], W[n // 2:], host.ACT_NONE)
+    assert h[0, 0] == 1 and h[0, 1] == 3 and h[0, -1] == 3 * K and int((h == 1).sum()) == n // 2 - 2
+
+
 @pytest.mark.parametrize("M,D,H", [(1, 513, 77), (16, 512, 4097), (17, 600, 5000), (33, 1000, 4096), (64, 31, 33), (64, 700, 5000)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
 @pytest.mark.parametrize("act", ["silu", "gelu", "relu2", "none"])
