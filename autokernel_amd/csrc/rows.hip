@@ -737,6 +737,15 @@ static ColPlan plan_cols(int64_t outer, int64_t red_n, int64_t inner, int kvec) 
   p.cg_log2 = 4;
   if (!p.vec) p.cg_log2 = 3;
   while (p.cg_log2 > 0 && (1 << (p.cg_log2 - 1)) >= groups) --p.cg_log2;
+  // More, up to 64, while that leaves 2048 blocks: every thread then has rows of its own to add where few
+  // rows leave row groups idle, and fewer sums to combine where there are many. Past 64 only for fewer rows
+  // than row groups. (us, one thread per output / 16 / as chosen: f16 sum over dim 0 of [5, 4000000] 17.7 /
+  // 31 / 12.1, [64, 4000000] 240 / 94 / 90, fp32 over dim 1 of [64, 8, 65536] 42 / 54 / 26, [1000, 2, 4096]
+  // 11.6 / 46 / 9.1; with 1024 blocks f16 [256, 262144] 22 / 26.)
+  if (p.vec && p.cg_log2 == 4)
+    while (p.cg_log2 < 8 && (p.cg_log2 < 6 || (kColThreads >> p.cg_log2) > red_n) &&
+           cdiv(groups, (int64_t)2 << p.cg_log2) * outer >= 2048)
+      ++p.cg_log2;
   p.col_blocks = cdiv(groups, (int64_t)1 << p.cg_log2);
   const int64_t rg = kColThreads >> p.cg_log2;
   const int64_t blocks = p.col_blocks * outer;

@@ -908,6 +908,22 @@ def test_reduce_strided_dim(gpu, shape, dim, dt):
     assert torch.equal(torch.isnan(m), torch.isnan(xn.max(dim).values))
 
 
+@pytest.mark.parametrize("shape,dim", [((2, 4200007), 0), ((3, 1048576), 0), ((5, 524296), 0), ((17, 524289), 0),
+                                       ((40, 2, 1100), 1), ((900, 3, 1100), 1), ((300, 130, 2100), 1), ((2100, 9, 516), 1)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32], ids=["f16", "f32"])
+def test_reduce_strided_dim_wide(gpu, shape, dim, dt):
+    """Few rows and many columns: 16, 32, 64, 128 and 256 column groups per block, ragged last blocks and
+    fewer rows than row groups. Bounds as in test_reduce_strided_dim."""
+    x = torch.randn(*shape, generator=torch.Generator().manual_seed(5)).to(dt)
+    n, xg = shape[dim], x.to(gpu)
+    y = kernels.get("reduce")(xg, dim)
+    exact = xg.double().sum(dim)
+    u = {torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dt]
+    bound = n * 2.0 ** -24 * xg.double().abs().sum(dim) + u * exact.abs() + (6e-8 if dt == torch.float16 else 1e-30)
+    assert bool(((y.double() - exact).abs() <= bound).all())
+    assert torch.equal(reduce_mod.reduce_max(xg, dim), xg.max(dim).values)
+
+
 def test_reduce_strided_dim_of_many_outputs(gpu):
     """A reduction whose column blocks would pass the 2^32 work-items of a grid (2^24 blocks of 256, here
     for 2^31 outputs of one row each) runs one thread per output."""
