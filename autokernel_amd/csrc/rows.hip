@@ -136,9 +136,12 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void layernorm_rows(
     float eps) {
   using G = RowGeom<L>;
   using R = RowRegs<T, L, VPT, ANY>;
-  // With rows of any alignment the affine parameters load after the reductions, aligned ones with the
-  // row (us, after / with the row: f16 [4096, 16385] 74 / 99, aligned [4096, 4096] 15.5 / 13.7).
-  constexpr bool kAfter = ANY;
+  // With rows of any alignment and on blocks of 1024 lanes, of which a CU holds one or two, the affine
+  // parameters load after the reductions, otherwise with the row (us, after / with the row: f16 [4096, 16385]
+  // 74 / 99, aligned f16 [1024, 32768] 26.6 / 31.1, fp32 [2048, 16384] 49.8 / 55.4, bf16 [1024, 65536] 58 / 148,
+  // whose 64 values a lane spill beside the parameters; but f16 [4096, 4096] 15.5 / 13.7, fp32 [4096, 4096]
+  // 24.2 / 20.5).
+  constexpr bool kAfter = ANY || L == 1024;
   __shared__ float red[G::kWPB];
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();

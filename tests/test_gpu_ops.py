@@ -953,6 +953,28 @@ def test_softmax_cross_entropy_of_the_widest_row(gpu):
         del y
 
 
+@pytest.mark.parametrize("cols", [4096, 8192, 16384, 16392, 32768, 32776, 65528, 65536])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+def test_layernorm_wide_aligned(gpu, cols, dt):
+    """Aligned rows on either side of a block of 1024 lanes (and of its two, four and eight vectors a
+    lane), the affine parameters loaded with the row or after it; with and without them. Bounds as in
+    test_row_ops_any_width_and_alignment."""
+    from autokernel_amd.kernels import _ops
+    g = torch.Generator().manual_seed(cols)
+    X, W, Bi = (torch.randn(*s, generator=g).to(dt).to(gpu) for s in ((5, cols), (cols,), (cols,)))
+    u = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dt]
+    Xd, n24 = X.double(), (cols + 16) * 2.0 ** -24
+    mean, var = Xd.mean(-1, keepdim=True), Xd.var(-1, unbiased=False, keepdim=True)
+    for w, b in ((W, Bi), (None, Bi), (W, None), (None, None)):
+        y = torch.empty_like(X)
+        _ops.layernorm(y, X, w, b, 1e-5)
+        h = (Xd - mean) / (var + 1e-5).sqrt() * (1 if w is None else w.double())
+        e = h if b is None else h + b.double()
+        slack = n24 * (Xd.abs().mean(-1, keepdim=True) / (var + 1e-5).sqrt() * (1 if w is None else w.double().abs()) + 2 * h.abs())
+        bound = u * e.abs() + 2 * slack + 8 * 2.0 ** -24 * (h.abs() + e.abs()) + (6e-8 if dt == torch.float16 else 1e-38)
+        assert bool(((y.double() - e).abs() <= bound).all()), (w is None, b is None)
+
+
 @pytest.mark.parametrize("cols", [3, 9, 1000, 4097, 32769, 65535, 65544, 70001, 131075])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
 def test_softmax_in_place(gpu, cols, dt):
