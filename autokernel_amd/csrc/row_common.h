@@ -16,8 +16,10 @@
 // take them twice, and both lanes store the same values). Measured, f16, us, against the kernels such
 // rows took before (2-byte loads in two or three passes, dword pairs, fp32-cached blocks): layernorm
 // [4097, 4097] 46.0 -> 16.8, rmsnorm 27 -> 15, row sums 15.4 -> 8.5; softmax [4096, 50257] 185 -> 157,
-// [4096, 20001] 92 -> 62, [16000, 1235] 37 -> 15; cross-entropy fp32 [4096, 20001] 144 -> 58. Widths just
-// under 65536, whose rows take straddling vectors, are level (softmax [1024, 65535] 62 -> 66).
+// [4096, 20001] 92 -> 62, [16000, 1235] 37 -> 15; cross-entropy fp32 [4096, 20001] 144 -> 58. Rows of
+// softmax and cross-entropy just under 65536 columns, whose pieces their lanes cannot hold, leave a few
+// elements at the row's start to one lane each (softmax [1024, 65535] 61.4 before, 63.6 with straddling vectors of their own, 57.8 so;
+// cross-entropy bf16 [300, 65535] 16.2, 19.5, 16.5).
 #pragma once
 #include <limits.h>
 
@@ -92,20 +94,23 @@ __device__ __forceinline__ void stv(void* p, const u32x4& v) {
 
 // The vectors of a row: vector idx holds elements off(idx) .. off(idx) + kVec - 1 and counts those
 // in [lo, hi) of them.
-template <typename T, bool ANY>
+// HEAD: see skew.
+template <typename T, bool ANY, bool HEAD = false>
 struct RowShape {
   int cols, nvec, skew;  // skew: elements between the aligned address at or before the row and its start
   // most: vectors the row's lanes hold. A row that an end piece would take past it (a width just under
-  // the widest one, or under 2^31) takes its vectors from its own start instead.
+  // the widest one, or under 2^31) takes its vectors from its own start instead, or (HEAD) from the first
+  // aligned address after it (skew < 0), which leaves head() elements, fewer than kVec, to the caller.
   __device__ __forceinline__ RowShape(const typename T::S* row, int cols_, bool active, int most = INT_MAX / T::kVec)
       : cols(cols_) {
     skew = ANY ? (int)(((uintptr_t)row & 15u) / sizeof(typename T::S)) : 0;
-    if (ANY && count() > most) skew = 0;
+    if (ANY && count() > most) skew = HEAD ? skew - T::kVec : 0;
     nvec = !active ? 0 : ANY ? count() : cols / T::kVec;
   }
   __device__ __forceinline__ int count() const {
     return (int)(((unsigned)cols + (unsigned)skew + T::kVec - 1) / T::kVec);
   }
+  __device__ __forceinline__ int head() const { return max(-skew, 0); }
   __device__ __forceinline__ int off(int idx) const {
     return ANY ? min(max(idx * T::kVec - skew, 0), cols - T::kVec) : idx * T::kVec;
   }
@@ -133,12 +138,13 @@ struct RowRegs {
 
   __device__ __forceinline__ static bool valid(int j, int gl, int nvec) { return gl + j * L < nvec; }
   // fn(element) for every element of vector j that counts (the vector must be valid)
-  template <typename F>
-  __device__ __forceinline__ void each(int j, int gl, const RowShape<T, ANY>& sh, F fn) const {
+  template <bool HEAD, typename F>
+  __device__ __forceinline__ void each(int j, int gl, const RowShape<T, ANY, HEAD>& sh, F fn) const {
     sh.each(gl + j * L, f + j * T::kVec, fn);
   }
 
-  __device__ __forceinline__ void load(const typename T::S* row, const RowShape<T, ANY>& sh, int gl) {
+  template <bool HEAD>
+  __device__ __forceinline__ void load(const typename T::S* row, const RowShape<T, ANY, HEAD>& sh, int gl) {
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const int idx = gl + j * L;
@@ -154,7 +160,8 @@ struct RowRegs {
   }
 
   // nt: nontemporal stores (outputs far larger than what a consumer could find in cache)
-  __device__ __forceinline__ void store(typename T::S* row, const RowShape<T, ANY>& sh, int gl, bool nt = false) const {
+  template <bool HEAD>
+  __device__ __forceinline__ void store(typename T::S* row, const RowShape<T, ANY, HEAD>& sh, int gl, bool nt = false) const {
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const int idx = gl + j * L;

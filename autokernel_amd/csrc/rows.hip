@@ -14,6 +14,7 @@ namespace ak {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kLoopThreads = 256;
+constexpr int kWidestRow = 65536;  // elements of a row cached in registers (1024 lanes of 64)
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -249,10 +250,12 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
+  constexpr bool kHead = ANY && L * VPT * T::kVec == kWidestRow;
+  const RowShape<T, ANY, kHead> sh(x + row * cols, cols, active, L * VPT);
+  const bool has_head = kHead && gl < sh.head();
   R r;
   r.load(x + row * cols, sh, gl);
-  float m = -INFINITY;
+  float h = has_head ? T::to_f(x[row * cols + gl]) : -INFINITY, m = h;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
     if (R::valid(j, gl, sh.nvec))
@@ -261,6 +264,7 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
   m = group_reduce<L, 1>(m, red);
   const float mb = m * kLog2e;
   float s = 0.f;
+  if (has_head) s = h = fast_exp2(__builtin_fmaf(h, kLog2e, -mb));
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     if (R::valid(j, gl, sh.nvec)) {
@@ -274,6 +278,7 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
 #pragma unroll
   for (int e = 0; e < R::kE; ++e) r.f[e] *= inv;
   r.store(y + row * cols, sh, gl, nt_out != 0);
+  if (has_head) y[row * cols + gl] = T::from_f(h * inv);
 }
 
 // Online (max, sum-of-exp) accumulator used by the looped softmax and cross-entropy kernels.
@@ -464,10 +469,13 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void ce_rows(
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  const RowShape<T, ANY> sh(x + row * cols, cols, active, L * VPT);
+  constexpr bool kHead = ANY && L * VPT * T::kVec == kWidestRow;
+  const RowShape<T, ANY, kHead> sh(x + row * cols, cols, active, L * VPT);
+  const bool has_head = kHead && gl < sh.head();
   R r;
   r.load(x + row * cols, sh, gl);
-  float m = -INFINITY;
+  const float h = has_head ? T::to_f(x[row * cols + gl]) : -INFINITY;
+  float m = h;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
     if (R::valid(j, gl, sh.nvec))
@@ -475,7 +483,7 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void ce_rows(
       for (int e = 0; e < T::kVec; ++e) m = fmaxf(m, r.f[j * T::kVec + e]);
   m = group_reduce<L, 1>(m, red);
   const float mb = m * kLog2e;
-  float s = 0.f;
+  float s = has_head ? fast_exp2(__builtin_fmaf(h, kLog2e, -mb)) : 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j)
     if (R::valid(j, gl, sh.nvec)) r.each(j, gl, sh, [&](float v) { s += fast_exp2(__builtin_fmaf(v, kLog2e, -mb)); });
