@@ -40,7 +40,9 @@ def gemm(A: torch.Tensor, B: torch.Tensor, out: torch.Tensor | None = None, spli
 
     split_k: let grids that leave most CUs idle split K (ak_gemm_ws); kernel_fn sets it. The model
     plug-in's projections keep the unsplit kernel, whose fp32 summation order reproduces stock
-    PyTorch's f16 logits bit for bit."""
+    PyTorch's f16 logits bit for bit with more than 64 rows. With at most 64 (short prompts, decode
+    steps) the K range is split over the waves of a block in any case (gemm_small.hip), an order of
+    its own: results are stock's to rounding."""
     return host._gemm(A, B, out=out, split_k=split_k)
 
 
