@@ -560,14 +560,29 @@ struct TileCfg {
   int bm, bn;
 };
 
+// One tile row (M <= 64) reads B once, so what counts is how much of it is in flight. A 64x96 or 64x128
+// tile has the CU to itself (four stages of LDS), two 64x64 ones share it and do not stop at each other's
+// barriers. Whether the wider tiles of an [N, K] B are the faster ones (us, 64x64 / 64x128): they are on
+// a grid well short of the CUs (1 x 20480 x 4096 38.1 / 33.1), or with many rows in the second round
+// (64 x 50304 x 1024 27.0 / 24.1); not on a full one (1 x 32000 x 4096 49.8 / 57.8, 64 x 32000 x 4096 57.2 /
+// 61.1) nor past two rounds (16 x 100000 x 2048 82 / 94). Of a [K, N] B, whose tile rows they make twice as
+// long, they are the faster ones up to two rounds (16 x 50304 x 4096 83 / 74) and for deep K past them (64 x
+// 100000 x 1024 57 / 51; but 64 x 100000 x 256 15.2 / 18.2). 128x192 tiles, two to a CU, waste more than half
+// of each on such rows and lose the same way (1 x 200000 x 768 55 / 66).
+static bool wide64_nt(int64_t M, int64_t N, int64_t K, int64_t waves) {
+  if (waves == 1) return N <= 24576 || K < 2048;
+  return waves == 2 && M > 32 && K >= 768;
+}
+
 // Pick the tile that keeps the 256 CUs busiest: fraction of CU-slots doing useful work over the
 // launch, weighted by the per-tile efficiency of smaller tiles (more LDS and L2 traffic per flop).
 // wide192: also consider 256x192 tiles (the LDS-DMA kernel with nn.Linear-layout B; 2048 x 6144,
 // a fused QKV projection, is then exactly one tile per CU). small64: also consider 64x64 tiles
 // (the same kernel, for grids that 128x128 tiles leave mostly idle) and 64x128 ones, and, with
 // nn.Linear-layout B, 64x96 and 128x192 (whose weight is eff192, see kPairK).
+// K: only for the rules of at most 64 rows.
 static TileCfg pick_tile(int64_t M, int64_t N, int nb, bool wide192 = false, bool small64 = false,
-                         int64_t batch = 1, double eff192 = 0.0) {
+                         int64_t batch = 1, double eff192 = 0.0, int64_t K = 0) {
   const TileCfg cands[] = {{256, 256}, {256, 128}, {128, 128}, {256, 192}, {64, 64}, {128, 192}, {64, 96}, {64, 128}};
   // relative per-flop throughput of the tiles (bf16, MI355X): 4096^3 on 256x256 1230 TF/s,
   // 2048x4096x4096 on 256x128 1084 TF/s, 2048x6144x4096 on 128x128 786 TF/s, on 256x192 1108 TF/s;
@@ -590,6 +605,8 @@ static TileCfg pick_tile(int64_t M, int64_t N, int nb, bool wide192 = false, boo
     const int bn = cands[i].bn / (nb == 2 ? 2 : 1);
     const int64_t tiles = cdiv(M, cands[i].bm) * cdiv(N, bn) * batch;
     const int64_t waves = cdiv(tiles, cus);
+    if (i == 5 && M <= 64 && waves > 1) continue;
+    if (i >= 6 && M <= 64 && !(wide192 ? wide64_nt(M, N, K, waves) : waves <= 2 || (M > 8 && K >= 768))) continue;
     const double used = (double)tiles / (double)(waves * cus);
     // padding waste inside edge tiles
     const double pad = (double)(M * N) / (double)(cdiv(M, cands[i].bm) * cands[i].bm * cdiv(N, bn) * bn);
@@ -719,7 +736,7 @@ static void launch_gemm_dma(const void* A, const void* B0, const void* B1, void*
                             int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, const EpiArgs& ep) {
   // 256x192 needs [N, K] B: a [K, N] B tile row of 192 elements does not split into 1 KB transfers
   constexpr bool kPair = NB == 1 && !BKN && EPI != kEpiPartial;
-  const TileCfg t = pick_tile(M, N, NB, !BKN, EPI != kEpiPartial, ep.batch, !kPair ? 0.0 : K <= kPairK ? kPairEff<EPI> : kLongEff192);
+  const TileCfg t = pick_tile(M, N, NB, !BKN, EPI != kEpiPartial, ep.batch, !kPair ? 0.0 : K <= kPairK ? kPairEff<EPI> : kLongEff192, K);
   if constexpr (NB == 1) {
     if constexpr (kPair) {
       if (t.bm == 128 && t.bn == 192) {

@@ -1439,6 +1439,24 @@ def test_gemm_bias_gelu_and_residual_epilogues(gpu, M, N, K):
         print(f"gemm bias+residual {M}x{N}x{K} {dt}: bit-equal", flush=True)
 
 
+@pytest.mark.parametrize("M,N,K,bt", [(1, 24576, 4096, True), (1, 24584, 4096, True), (64, 20480, 2048, True), (64, 32000, 2048, True),
+                                      (64, 50304, 768, True), (33, 50304, 768, True), (32, 50304, 768, True), (16, 100000, 64, True),
+                                      (9, 100000, 768, False), (8, 100000, 768, False), (64, 50304, 512, False), (40, 100000, 256, False)])
+def test_gemm_tiles_of_few_rows(gpu, M, N, K, bt):
+    """At most 64 rows against many columns, on both sides of the rules that choose among 64-row tiles:
+    the bits of the register-staged kernel (every tile sums each output's products in the same order),
+    which the same values take as the first rows of a 65-row product in rows padded by one element."""
+    from autokernel_amd.kernels import _ops
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(65, K, generator=g).half().to(gpu)
+    B = (torch.randn(*((N, K) if bt else (K, N)), generator=g) * 0.1).half().to(gpu)
+    got, want = torch.empty(M, N, device=gpu, dtype=torch.float16), torch.empty(65, N, device=gpu, dtype=torch.float16)
+    _ops.gemm(got, A[:M], B, bt)
+    A2, B2 = (torch.nn.functional.pad(t, (0, 1))[:, :-1] for t in (A, B))
+    _ops.gemm(want, A2, B2, bt)
+    assert torch.equal(got, want[:M])
+
+
 @pytest.mark.parametrize("M,N,K,bt", [
     (2047, 2305, 64, True), (2048, 2304, 768, True), (1000, 5000, 1024, True), (8191, 767, 128, True),  # 128x192
     (500, 11000, 1088, True), (511, 2300, 320, True), (2048, 768, 192, True), (65, 96, 64, True),  # 128x192, 64x96, 64x64
