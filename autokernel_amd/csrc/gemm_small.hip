@@ -124,7 +124,7 @@ __global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typen
     typename SV::R n[BT ? 1 : U][NB][BT ? 1 : KV];
   };
   auto load = [&](int k0, Group& x) {
-    if (k0 + U * KS <= K) {  // uniform
+    if (K - k0 >= U * KS) {  // uniform (k0 + U * KS may pass an int)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = k0 + u * KS;

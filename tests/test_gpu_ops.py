@@ -388,6 +388,22 @@ def test_matmul_few_rows_of_many_columns(gpu, dt, K):
     assert h[0, 0] == 1 and h[0, 1] == 3 and h[0, -1] == 3 * K and int((h == 1).sum()) == n // 2 - 2
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_matmul_few_rows_of_the_deepest_k(gpu, dt):
+    """One row and one column of 2^31 - 1 values, whose last group of k ends past an int: its elements are
+    loaded one by one, and the sum has the first and the last product."""
+    from autokernel_amd.kernels import _ops
+    if torch.cuda.mem_get_info()[0] < 24 << 30:
+        pytest.skip("needs 17 GB")
+    k = 2 ** 31 - 1
+    a, b = (torch.zeros(k, dtype=dt, device=gpu) for _ in range(2))
+    a[0], a[-1], b[0], b[-1] = 2, 3, 5, 7
+    for bt in (True, False):
+        c = torch.empty(1, 1, dtype=dt, device=gpu)
+        _ops.gemm(c, a.view(1, k), b.view(1, k) if bt else b.view(k, 1), bt)
+        assert float(c) == 31, bt
+
+
 @pytest.mark.parametrize("M,D,H", [(1, 513, 77), (16, 512, 4097), (17, 600, 5000), (33, 1000, 4096), (64, 31, 33), (64, 700, 5000)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
 @pytest.mark.parametrize("act", ["silu", "gelu", "relu2", "none"])
