@@ -739,8 +739,13 @@ struct ColPlan {
 
 static ColPlan plan_cols(int64_t outer, int64_t red_n, int64_t inner, int kvec) {
   ColPlan p{};
-  // Blocks of the column kernel would be nearly empty, and one thread per output already fills the chip.
-  p.short_rows = red_n * inner < 4096 && outer * inner >= 65536;
+  // Blocks of the column kernel would be nearly empty, and one thread per output already fills the chip; or
+  // the call is small and one thread adds its few rows before a block has combined its row groups (us, one
+  // thread per output / column blocks: f16 [2, 300000] 2.8 / 5.0, [8, 300000] 3.4 / 5.0, [16, 262144] 4.1 /
+  // 4.7, [3, 542] 2.6 / 3.1, fp32 [2, 1000000] 4.5 / 5.2; but [13, 262144] 6.0 / 5.1, [16, 16384] 3.7 / 3.1,
+  // f16 [8, 1000000] 8.1 / 7.0).
+  p.short_rows = (red_n * inner < 4096 && outer * inner >= 65536) ||
+                 (red_n <= (outer * inner >= 131072 ? 16 : 12) && red_n * outer * inner < (13 << 16) * (int64_t)kvec);
   p.vec = inner >= kvec;
   const int64_t groups = p.vec ? cdiv(inner, kvec) : inner;
   // 16 column groups (256 bytes of a row) per block; fewer for narrower rows, so that the block's

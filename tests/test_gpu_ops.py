@@ -925,11 +925,13 @@ def test_reduce_strided_dim(gpu, shape, dim, dt):
 
 
 @pytest.mark.parametrize("shape,dim", [((2, 4200007), 0), ((3, 1048576), 0), ((5, 524296), 0), ((17, 524289), 0),
-                                       ((40, 2, 1100), 1), ((900, 3, 1100), 1), ((300, 130, 2100), 1), ((2100, 9, 516), 1)])
+                                       ((40, 2, 1100), 1), ((900, 3, 1100), 1), ((300, 130, 2100), 1), ((2100, 9, 516), 1),
+                                       ((12, 500), 0), ((13, 500), 0), ((16, 131080), 0), ((17, 131080), 0), ((2, 3000000), 0)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32], ids=["f16", "f32"])
 def test_reduce_strided_dim_wide(gpu, shape, dim, dt):
     """Few rows and many columns: 16, 32, 64, 128 and 256 column groups per block, ragged last blocks and
-    fewer rows than row groups. Bounds as in test_reduce_strided_dim."""
+    fewer rows than row groups; and on both sides of the calls that run one thread per output. Bounds as in
+    test_reduce_strided_dim."""
     x = torch.randn(*shape, generator=torch.Generator().manual_seed(5)).to(dt)
     n, xg = shape[dim], x.to(gpu)
     y = kernels.get("reduce")(xg, dim)
