@@ -700,10 +700,11 @@ static void launch_dma_cfg(const void* A, const void* B0, const void* B1, void* 
   // then exposed; measured 2048x1024x4096: 50.9 us against 59.0 us two-stage). With more tiles the
   // 64-deep pair is faster per tile (2048x6144x4096 on 192 tiles of 256x256: 109.9 us against
   // 127.5 us).
-  // 64x64 tiles keep their four 64-deep stages there (f16: 128x768x768 7.3 us 32-deep, 6.3 64-deep;
-  // 512x768x3072 23.1, 17.4).
-  constexpr bool kOk32 = P::kOk32 && BM > 64;
-  if (kOk32 && 2 * tiles_m * tiles_n * ep.splits * ep.batch <= kCUs) {
+  // 64-row tiles keep their four 64-deep stages there (f16: 128x768x768 7.3 us 32-deep, 6.3 64-deep;
+  // 512x768x3072 23.1, 17.4) unless K is so short that most of what they fetch is past it (12x128x64 nn 2.95,
+  // 3.15; 112x1344x64 nn 3.36, 3.59).
+  constexpr bool kOk32 = P::kOk32;
+  if (kOk32 && (BM > 64 || K <= 128) && 2 * tiles_m * tiles_n * ep.splits * ep.batch <= kCUs) {
     if constexpr (kOk32)
       launch_dma_kernel<T, BM, BN, WM, WN, NB, EPI, 32, 4, BKN>(A, B0, B1, C, M, N, K, lda, ldb, ldc, tiles_m,
                                                                 tiles_n, s, ep);

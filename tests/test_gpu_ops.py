@@ -1478,6 +1478,7 @@ def test_gemm_tiles_of_few_rows(gpu, M, N, K, bt):
 @pytest.mark.parametrize("M,N,K,bt", [
     (2047, 2305, 64, True), (2048, 2304, 768, True), (1000, 5000, 1024, True), (8191, 767, 128, True),  # 128x192
     (500, 11000, 1088, True), (511, 2300, 320, True), (2048, 768, 192, True), (65, 96, 64, True),  # 128x192, 64x96, 64x64
+    (100, 1344, 128, True), (100, 1344, 64, False),  # 64x64 in 32-deep stages
     (2047, 1000, 1088, True), (2047, 1000, 1088, False), (511, 4096, 64, False),  # 64x128
     # rows at odd offsets: 256x256, 256x192, 128x128, 128x192, 64x128, 64x64
     (4095, 4095, 1088, True), (2047, 6143, 1088, True), (2047, 2047, 1088, True), (500, 10999, 1088, True),
