@@ -66,10 +66,45 @@ __device__ __forceinline__ u32x4 load_kchunk(const uint16_t* __restrict__ p, int
   }
 }
 
+// gemm_small's order of the sums (N <= 4096), for tiles of a batch of such products: slice i is k-groups i,
+// i + 16, ..., and the slices' sums are added as a tree over 16 waves adds them. With the slices visited in
+// bit-reversed order each pair of the tree is complete before the next begins, so four held tiles are enough.
+struct SliceWalk {
+  int g = 0, i = 0;  // group, position of its slice (16: past the end)
+  __device__ __forceinline__ void step(int groups) {
+    for (g += 16; g >= groups && i < 16;) {
+      ++i;
+      g = (int)(__builtin_bitreverse32((unsigned)i) >> 28);
+    }
+  }
+};
+// The slice at position i is in acc: hold it (acc starts the next) or add it to the held left halves it ends.
+// Level d of part holds 2^d slices. (In LDS, or with the walk unrolled, the tiles were slower.)
+template <int FM, int FN>
+__device__ __forceinline__ void end_slice(int i, f32x4 (&part)[4][FM][FN], f32x4 (&acc)[FM][FN]) {
+  bool held = false;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    if (held) continue;
+    held = ((i >> d) & 1) == 0;  // uniform
+#pragma unroll
+    for (int x = 0; x < FM; ++x)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        if (held) {
+          part[d][x][j] = acc[x][j];
+          acc[x][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        } else {
+          acc[x][j] = part[d][x][j] + acc[x][j];
+        }
+      }
+  }
+}
+
 // --------------------------------------------------------------------------------------------
-// The f16 / bf16 kernel
+// The f16 / bf16 kernel. SL: 0, or the depth of a k-group (32 or 64) summed in gemm_small's order.
 // --------------------------------------------------------------------------------------------
-template <typename T, bool BT, bool VEC, int BM, int BN, int WM, int WN, int NB, int EPI>
+template <typename T, bool BT, bool VEC, int BM, int BN, int WM, int WN, int NB, int EPI, int SL = 0>
 __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
     uint16_t* __restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
@@ -85,6 +120,9 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
 
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * kBK];
   __shared__ __attribute__((aligned(16))) uint16_t sB[2][NB][BN * kBK];
+  if constexpr (SL != 0) {
+    if (skip_item(ep)) return;
+  }
   batch_bases(A, B0, C, ep);
 
   int tm, tn;
@@ -101,12 +139,14 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
   u32x4 rbt[NB][BT ? BT_CH : 1];
   u32x4 rbn[BT ? 1 : BN_U][4];
 
-  auto gload = [&](int k0) {
+  // The tile's halves of 32 are k0 .. and k1 .. (k0 + 32 unless SL is 32).
+  auto gload = [&](int k0, int k1) {
+    auto at = [&](int p) { return SL == 32 && p >= 32 ? k1 + p - 32 : k0 + p; };
 #pragma unroll
     for (int i = 0; i < A_CH; ++i) {
       const int q = tid + i * kThreads;
       const int row = q / kKC, c = q % kKC;
-      ra[i] = load_kchunk<VEC>(A, lda, m0 + row, M, k0 + c * 8, K);
+      ra[i] = load_kchunk<VEC>(A, lda, m0 + row, M, at(c * 8), K);
     }
     if constexpr (BT) {
 #pragma unroll
@@ -115,7 +155,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
         for (int i = 0; i < BT_CH; ++i) {
           const int q = tid + i * kThreads;
           const int row = q / kKC, c = q % kKC;
-          if (q < BN * kKC) rbt[b][i] = load_kchunk<VEC>(Bm[b], ldb, n0 + row, N, k0 + c * 8, K);
+          if (q < BN * kKC) rbt[b][i] = load_kchunk<VEC>(Bm[b], ldb, n0 + row, N, at(c * 8), K);
         }
     } else {
 #pragma unroll
@@ -126,7 +166,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
         if (u < BN_UNITS) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int k = k0 + kq * 4 + r;
+            const int k = at(kq * 4) + r;
             const int n = n0 + ng * 8;
             u32x4 v = {0u, 0u, 0u, 0u};
             if (k < K) {
@@ -187,8 +227,24 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int KT = (K + kBK - 1) / kBK;
-  gload(0);
+  const int groups = SL ? (K + SL - 1) / (SL ? SL : 1) : 0;
+  const int KT = SL == 32 ? (groups + 1) / 2 : (K + kBK - 1) / kBK;
+  f32x4 part[4][SL ? FM : 1][SL ? FN : 1];
+  SliceWalk fetch, use;
+  auto take = [&]() {  // the next group's k; past the last one K, whose loads are zeros
+    const int k = fetch.i < 16 ? fetch.g * SL : K;
+    fetch.step(groups);
+    return k;
+  };
+  auto load_tile = [&](int kt) {
+    if constexpr (SL) {
+      const int k0 = take();
+      gload(k0, SL == 32 ? take() : k0 + 32);
+    } else {
+      gload(kt * kBK, kt * kBK + 32);
+    }
+  };
+  load_tile(0);
   sstore(0);
   __syncthreads();
 
@@ -196,7 +252,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
   const int fc = lane >> 4;        // 8-element k group inside a 32-k step
   for (int kt = 0; kt < KT; ++kt) {
     const int cur = kt & 1;
-    if (kt + 1 < KT) gload((kt + 1) * kBK);
+    if (kt + 1 < KT) load_tile(kt + 1);
 #pragma unroll
     for (int s = 0; s < kBK / 32; ++s) {
       u32x4 fa[FM], fb[NB][FN];
@@ -218,6 +274,13 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
         for (int i = 0; i < FM; ++i)
 #pragma unroll
           for (int j = 0; j < FN; ++j) acc[b][i][j] = mfma16x16x32<T>(fb[b][j], fa[i], acc[b][i][j]);
+      if constexpr (SL != 0) {
+        if (SL == 32 || s == 1) {
+          int i = use.i;
+          use.step(groups);
+          for (; i < use.i; ++i) end_slice<FM, FN>(i, part, acc[0]);
+        }
+      }
     }
     if (kt + 1 < KT) sstore(cur ^ 1);
     __syncthreads();
@@ -304,7 +367,8 @@ struct DmaB {
   static constexpr int kRows = BKN ? BKD : BN;   // tile rows per stage
 };
 
-template <typename T, int BM, int BN, int WM, int WN, int NB, int BKD, int NS, bool BKN, int MF>
+// SL: the k-tiles are the groups of gemm_small's order.
+template <typename T, int BM, int BN, int WM, int WN, int NB, int BKD, int NS, bool BKN, int MF, bool SL>
 __device__ __forceinline__ void gemm_dma_ns_kloop(
     typename MfmaAcc<MF>::type (&acc)[NB][BM / WM / MF][BN / WN / MF], const uint16_t* A, const uint16_t* B0,
     const uint16_t* B1, const uint32_t* oa, const uint32_t* ob, uint32_t kb_step_b, int K, int wid,
@@ -326,7 +390,16 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
   const int fr = lane & (MF - 1), fc = lane / MF;
   uint16_t* const st[4] = {s0, s1, s2, s3};
 
+  const int KT = K / BKD;
+  f32x4 part[4][SL ? FM : 1][SL ? FN : 1];
+  SliceWalk fetch, use;
   auto issue = [&](int kt, uint16_t* sp) {
+    if constexpr (SL) {  // issues come in the tiles' order; past the end the last one again
+      kt = fetch.g;
+      SliceWalk n = fetch;
+      n.step(KT);
+      if (n.i < 16) fetch = n;
+    }
     const uint32_t kb = 2u * (uint32_t)(kt * BKD);
     const uint32_t kbb = BKN ? (uint32_t)kt * kb_step_b : kb;
 #pragma unroll
@@ -373,7 +446,6 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[b][i][j] = mfma_tile<T, MF>(fb[b][j], fa[i], acc[b][i][j]);
   };
-  const int KT = K / BKD;
   // One k-step: first half of the MFMAs; at a tile's last step (cross) wait until the next tile
   // has landed (NS - 2 later tiles may still be in flight), barrier (every wave holds this tile's
   // fragments, so its stage is free) and refill the stage with tile refill_kt (clamped: past the
@@ -411,6 +483,11 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
         for (int s = 0; s < STEPS; ++s) {
           if (s + 1 < STEPS) kstep(st[u], s + 1, false, st[u], 0);
           else kstep(st[(u + 1) % NS], 0, true, st[u], min(t + NS, KT - 1));
+        }
+        if constexpr (SL) {
+          int i = use.i;
+          use.step(KT);
+          for (; i < use.i; ++i) end_slice<FM, FN>(i, part, acc[0]);
         }
       }
     }
@@ -464,7 +541,7 @@ __device__ __forceinline__ void store_tile_rows(uint16_t* __restrict__ C, int64_
   }
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int MF, int OCC>
+template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int MF, int OCC, bool SL>
 __global__ __launch_bounds__(WM* WN* kWave, OCC* WM* WN / 4) void gemm_dma(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B0, const uint16_t* __restrict__ B1,
     uint16_t* __restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
@@ -539,7 +616,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC* WM* WN / 4) void gemm_dma(
 #pragma unroll
         for (int e = 0; e < (int)(sizeof(Acc) / 4); ++e) acc[b][i][j][e] = 0.f;
 
-  gemm_dma_ns_kloop<T, BM, BN, WM, WN, NB, BKD, NS, BKN, MF>(acc, A, B0, B1, oa, ob, kb_step_b, K, wid, wm, wn,
+  gemm_dma_ns_kloop<T, BM, BN, WM, WN, NB, BKD, NS, BKN, MF, SL>(acc, A, B0, B1, oa, ob, kb_step_b, K, wid, wm, wn,
                                                              lane, sS0, sS1, sS2, sS3);
 
   // 16x16 fragment: lane holds C[m0' + lane % 16][n0' + 4 (lane / 16) + 0..3]
@@ -656,13 +733,13 @@ static void launch_gemm_tiled(const void* A, const void* B0, const void* B1, voi
 constexpr int kCUs = 256;  // MI355X compute units
 
 // OCC: blocks that must fit on a CU together (it bounds the registers; LDS has to fit as well).
-template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int OCC = 1>
+template <typename T, int BM, int BN, int WM, int WN, int NB, int EPI, int BKD, int NS, bool BKN, int OCC = 1, bool SL = false>
 static void launch_dma_kernel(const void* A, const void* B0, const void* B1, void* C, int M, int N, int K,
                               int64_t lda, int64_t ldb, int64_t ldc, int tiles_m, int tiles_n, hipStream_t s,
                               const EpiArgs& ep) {
   // MFMA shape 16x16x32 (32x32x16 fragments measured 4-10 % slower on every workload)
   constexpr int MF = 16;
-  gemm_dma<T, BM, BN, WM, WN, NB, EPI, BKD, NS, BKN, MF, OCC><<<dim3(tiles_m * tiles_n, ep.splits, ep.batch), WM * WN * kWave, 0, s>>>(
+  gemm_dma<T, BM, BN, WM, WN, NB, EPI, BKD, NS, BKN, MF, OCC, SL><<<dim3(tiles_m * tiles_n, ep.splits, ep.batch), WM * WN * kWave, 0, s>>>(
       (const uint16_t*)A, (const uint16_t*)B0, (const uint16_t*)B1, (uint16_t*)C, M, N, K, lda, ldb, ldc,
       tiles_m, tiles_n, ep);
 }
@@ -780,6 +857,45 @@ static void launch_gemm_dma(const void* A, const void* B0, const void* B1, void*
   }
 }
 
+// A batch of products that each take gemm_small, summed in its order by tiles: past 512 blocks of 32 x 32 the
+// tiles, which share their operands' loads, are the faster form (us, a block's 16 waves / four slices a wave / these:
+// f16 nt 64 x 64 x 512, 64 items 12.4 / 7.5 / 10.2, 512 items 76 / 27 / 17; 64 x 1024 x 1024, 4 items 15 / 8 / 13, 128 items 425 /
+// 137 / 72; nn 32 x 3000 x 1000, 8 items 33 / 38 / 26). dma: the LDS-DMA kernel reads them; vec: 16-byte loads do.
+template <typename T>
+static int launch_gemm_slices(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
+                              int64_t ldc, bool bt, bool dma, bool vec, hipStream_t s, const EpiArgs& ep) {
+  const int tm = (int)cdiv(M, 64), tn = (int)cdiv(N, 64);
+  if (!dma) {
+#define AK_SL(BT, VEC, SL)                                                                                       \
+  gemm_mfma<T, BT, VEC, 64, 64, 2, 2, 1, kEpiStore, SL><<<dim3(tm * tn, 1, ep.batch), 4 * kWave, 0, s>>>(        \
+      (const uint16_t*)A, (const uint16_t*)B, nullptr, (uint16_t*)C, M, N, K, lda, ldb, ldc, tm, tn, ep)
+#define AK_SLV(BT, SL)              \
+  {                                 \
+    if (vec) AK_SL(BT, true, SL);   \
+    else AK_SL(BT, false, SL);      \
+  }
+    if (small_k64(M, N, bt)) {
+      if (bt) AK_SLV(true, 64) else AK_SLV(false, 64)
+    } else {
+      if (bt) AK_SLV(true, 32) else AK_SLV(false, 32)
+    }
+#undef AK_SLV
+#undef AK_SL
+    return record_launch();
+  }
+#define AK_SL(BKD, BKN) \
+  launch_dma_kernel<T, 64, 64, 2, 2, 1, kEpiStore, BKD, 4, BKN, 2, true>(A, B, nullptr, C, M, N, K, lda, ldb, ldc, tm, tn, s, ep)
+  if (small_k64(M, N, bt)) {
+    if (bt) AK_SL(64, false);
+    else AK_SL(64, true);
+  } else {
+    if (bt) AK_SL(32, false);
+    else AK_SL(32, true);
+  }
+#undef AK_SL
+  return record_launch();
+}
+
 // Products of at most kSmallM rows on operands the LDS-DMA kernel can read: whether gemm_small is the
 // faster one. Measured (bf16, three rotating operand sets, us, LDS-DMA unsplit / gemm_small, M = 1, 16,
 // 32, 64; "nt" is an [N, K] B):
@@ -807,10 +923,10 @@ static bool dma_shape(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
 // The period of a batch's kernel choice. A product of at most kSmallM rows that small_rows_win leaves to
 // the LDS-DMA kernel takes gemm_small where its operands are off 16 bytes, and the two sum in different
 // orders. Every item of a batch has to equal its 2-D product, so where the batch strides move items on
-// and off 16 bytes, items z, z + p, ... are one launch.
+// and off 16 bytes, the aligned ones (z, z + p, ... for one z) are a launch of their own.
 static int64_t batch_period(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t stride_a,
                             int64_t stride_b, bool bt) {
-  if (M > kSmallM || !dma_shape(M, N, K, lda, ldb, bt) || small_rows_win(M, N, K, bt, 1)) return 1;
+  if (M > kSmallM || N > small_max_n(1) || !dma_shape(M, N, K, lda, ldb, bt) || small_rows_win(M, N, K, bt, 1)) return 1;
   int64_t p = 1;
   while ((p * stride_a) % 8 != 0 || (p * stride_b) % 8 != 0) p *= 2;
   return p;
@@ -824,12 +940,19 @@ static int launch_gemm16(const void* A, const void* B0, const void* B1, void* C,
   // residual (B1 of one product): the epilogue checks each 8-byte access. They must not choose the kernel
   // either, whose order of the sums an epilogue shares with the plain product.
   bool vec = K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && (bt || N % 8 == 0) && host_aligned16(A) && host_aligned16(B0) &&
-             (NB == 1 || host_aligned16(B1));
+             (NB == 1 || host_aligned16(B1)) && ep.skip < 0;
   const int m = (int)M, n = (int)N, k = (int)K;
   const bool dma = vec && dma_shape(M, N, K, lda, ldb, bt);
   // Few rows: always for operands that path cannot read, by shape for those it can.
-  if (M <= kSmallM && N <= small_max_n(NB) && K > 0 && (bt || NB == 1) && (!dma || small_rows_win(M, N, K, bt, NB)))
+  if (M <= kSmallM && N <= small_max_n(NB) && K > 0 && (bt || NB == 1) && (!dma || small_rows_win(M, N, K, bt, NB))) {
+    if constexpr (NB == 1 && EPI == kEpiStore) {
+      if (ep.batch > 1 && M > 16 && N <= 4096 && K <= (1 << 30) && cdiv(M, 32) * cdiv(N, 32) * ep.batch >= 512) {
+        const bool vz = vec && ep.batch_a % 8 == 0 && ep.batch_b % 8 == 0;
+        return launch_gemm_slices<T>(A, B0, C, m, n, k, lda, ldb, ldc, bt, dma && vz, vz, s, ep);
+      }
+    }
     return launch_gemm_small<T, NB, EPI>(A, B0, B1, C, M, N, K, lda, ldb, ldc, bt, s, ep);
+  }
   vec = vec && ep.batch_a % 8 == 0 && ep.batch_b % 8 == 0;
   if (bt && dma && vec) {
     launch_gemm_dma<T, NB, EPI, false>(A, B0, B1, C, m, n, k, lda, ldb, ldc, s, ep);
@@ -967,16 +1090,22 @@ extern "C" int ak_gemm_batched(int dtype, const void* A, const void* B, void* C,
   const bool bt = b_trans != 0;
   const int esz = dtype == AK_F32 ? 4 : 2;
   const int64_t period = dtype == AK_F32 ? 1 : batch_period(M, N, K, lda, ldb, stride_a, stride_b, bt);
-  const int64_t sa = stride_a * period, sb = stride_b * period, sc = stride_c * period;
-  // grid z holds at most 65535 items: larger batches run in chunks
-  constexpr int64_t kMaxZ = 65535;
-  for (int64_t r = 0; r < period && r < batch; ++r) {
-    const int64_t items = cdiv(batch - r, period);
+  // the items both of whose operands are aligned: one of the first `period`, and every period-th after it
+  int64_t own = -1;
+  if (period > 1)
+    for (int64_t z = 0; z < period && own < 0; ++z)
+      if (host_aligned16((const char*)A + z * stride_a * esz) && host_aligned16((const char*)B + z * stride_b * esz)) own = z;
+  // items first, first + step, ...; skip: leave the aligned ones out
+  auto launch = [&](int64_t first, int64_t step, bool skip) -> int {
+    const int64_t sa = stride_a * step, sb = stride_b * step, sc = stride_c * step;
+    // grid z holds at most 65535 items: larger batches run in chunks
+    constexpr int64_t kMaxZ = 65535;
+    const int64_t items = cdiv(batch - first, step);
     for (int64_t z0 = 0; z0 < items; z0 += kMaxZ) {
-      const int64_t nz = items - z0 < kMaxZ ? items - z0 : kMaxZ, first = r + z0 * period;
-      const char* a = (const char*)A + first * stride_a * esz;
-      const char* b = (const char*)B + first * stride_b * esz;
-      char* c = (char*)C + first * stride_c * esz;
+      const int64_t nz = items - z0 < kMaxZ ? items - z0 : kMaxZ, z = first + z0 * step;
+      const char* a = (const char*)A + z * stride_a * esz;
+      const char* b = (const char*)B + z * stride_b * esz;
+      char* c = (char*)C + z * stride_c * esz;
       int st = AK_OK;
       if (dtype == AK_F32) {
         st = launch_gemm32(a, b, c, M, N, K, lda, ldb, ldc, bt, stream, (int)nz, sa, sb, sc);
@@ -986,14 +1115,21 @@ extern "C" int ak_gemm_batched(int dtype, const void* A, const void* B, void* C,
         ep.batch_a = sa;
         ep.batch_b = sb;
         ep.batch_c = sc;
+        if (skip) {
+          ep.skip = (int)((own + period - z0 % period) % period);
+          ep.skip_period = (int)period;
+        }
         if (dtype == AK_F16) st = launch_gemm16<TF16, 1, kEpiStore>(a, b, nullptr, c, M, N, K, lda, ldb, ldc, bt, stream, ep);
         else if (dtype == AK_BF16) st = launch_gemm16<TBF16, 1, kEpiStore>(a, b, nullptr, c, M, N, K, lda, ldb, ldc, bt, stream, ep);
         else return AK_EINVAL;
       }
       if (st != AK_OK) return st;
     }
-  }
-  return AK_OK;
+    return AK_OK;
+  };
+  if (own < 0 || own >= batch) return launch(0, 1, false);
+  const int st = launch(own, period, false);
+  return st == AK_OK && batch > 1 ? launch(0, 1, true) : st;
 }
 
 extern "C" int64_t ak_gemm_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

@@ -60,7 +60,14 @@ struct EpiArgs {
   // the operand across the batch).
   int batch = 1;
   int64_t batch_a = 0, batch_b = 0, batch_c = 0;
+  // Items skip, skip + skip_period, ... are another launch's (their operands are 16-byte aligned, the others'
+  // are not); -1: none.
+  int skip = -1, skip_period = 1;
 };
+
+__device__ __forceinline__ bool skip_item(const EpiArgs& ep) {
+  return ep.skip >= 0 && (int)blockIdx.z % ep.skip_period == ep.skip;
+}
 
 // Bases of this block's batch item (grid z); one item when ep.batch == 1.
 template <class PA, class PB, class PC>
@@ -298,6 +305,13 @@ __device__ __forceinline__ void tile_epilogue(uint16_t* __restrict__ C, const ui
 // 2^32 work-items of a grid: at most 16 per column (32 for gate/up).
 constexpr int64_t kSmallM = 64;
 constexpr int64_t small_max_n(int nb) { return ((int64_t)1 << 28) / nb - 64; }
+// gemm_small for one product of N <= 4096 columns: whether its waves take groups of two k-steps (of one
+// else), and its blocks.
+inline bool small_k64(int64_t M, int64_t N, bool bt) { return M <= 16 || N <= 1024 || (bt && M <= 32); }
+inline int64_t small_blocks(int64_t M, int64_t N, bool bt) {
+  const bool one = M <= 16 || N <= 1024;  // 16 rows a block
+  return cdiv(M, one ? 16 : 32) * cdiv(N, bt && (one || M <= 32) ? 16 : 32);
+}
 template <typename T, int NB, int EPI>
 int launch_gemm_small(const void* A, const void* B0, const void* B1, void* C, int64_t M, int64_t N, int64_t K,
                       int64_t lda, int64_t ldb, int64_t ldc, bool bt, hipStream_t s, const EpiArgs& ep);

@@ -18,10 +18,11 @@
 // Measured (us, before / now; three rotating operand sets): bf16 nt 1 x 4096 x 4096 13.9 / 9.4, 16 x 4096 x
 // 11008 30 / 26, nn 29 x 3702 x 10112 (repacked before) 237 / 64, nn 10 x 1536 x 246 28 / 12; gate/up
 // 16 x 4096 -> 11008 65 / 55; f32 nt 16 x 11008 x 4096 563 / 57, nn 28 x 553 x 6656 940 / 53.
-// WV and U, which fix the order of the sums, depend on M, N, K, B's layout and NB only, so that a batched
+// The slices (WV, or WV LV) and U, which fix the order of the sums, depend on M, N, B's layout and NB only, so that a batched
 // product equals its items, and an epilogue equals the separate op, bit for bit. Which products come here
 // also depends on the alignment of A and B (launch_gemm16), which a product and its epilogue forms share;
-// ak_gemm_batched launches items of different alignment apart (batch_period).
+// ak_gemm_batched launches the aligned items of a batch apart where that decides (batch_period), and large
+// batches run in the same order on other kernels (launch_gemm_small, launch_gemm_slices).
 #include <limits.h>
 
 #include "gemm_common.h"
@@ -77,12 +78,14 @@ __device__ __forceinline__ typename SmallVec<S, VN>::R small_load_n(const S* p, 
 }
 
 // Waves per SIMD the registers allow without spills.
-constexpr int small_occupancy(int wv, int mf, bool bt, bool f32) {
-  return wv == 16 || (bt && (mf == 1 || (mf == 4 && !f32))) ? 4 : bt && mf == 2 ? 3 : 2;
+constexpr int small_occupancy(int wv, int lv, int mf, bool bt, bool f32) {
+  return lv > 1 ? 2 : wv == 16 || (bt && (mf == 1 || (mf == 4 && !f32))) ? 4 : bt && mf == 2 ? 3 : 2;
 }
 
-template <typename T, bool BT, int NB, int EPI, int MF, int CF, int WV, int U>
-__global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typename T::S) == 4)) void gemm_small(
+// LV: the K slices of a wave. With LV = 1 wave w adds slice w; with more it adds slices w, w + WV, ... one
+// after another and puts them together in registers in the order the tree over WV LV waves would.
+template <typename T, bool BT, int NB, int EPI, int MF, int CF, int WV, int LV, int U>
+__global__ __launch_bounds__(WV* kWave, small_occupancy(WV, LV, MF, BT, sizeof(typename T::S) == 4)) void gemm_small(
     const typename T::S* __restrict__ A, const typename T::S* __restrict__ B0, const typename T::S* __restrict__ B1,
     typename T::S* __restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, EpiArgs ep) {
   using S = typename T::S;
@@ -98,6 +101,7 @@ __global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typen
   constexpr int kTile = MF * 16 * (BNC + 4);
   constexpr int kTree = WV / 2 * kFrag * kParts * 256;
   __shared__ __attribute__((aligned(16))) float lds[kTree > NB * kTile ? kTree : NB * kTile];
+  if (skip_item(ep)) return;
   batch_bases(A, B0, C, ep);
   const int n0 = blockIdx.x * BNC, m0 = blockIdx.y * (MF * 16);
   const int lane = lane_id(), w = wave_id();
@@ -213,9 +217,87 @@ __global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typen
           }
         }
   };
-  constexpr int kGroup = U * KS, kStride = WV * kGroup;
+  // s + o; fp32: with what the total lost (two-sum) added to both compensations
+  auto add = [&](f32x4& s, f32x4& sc, const f32x4& o, const f32x4& oc) {
+    if constexpr (F32) {
+      const f32x4 t = s + o, z = t - s;
+      sc += oc + ((s - (t - z)) + (o - z));
+      s = t;
+    } else {
+      s += o;
+    }
+  };
+  constexpr int kGroup = U * KS, kStride = WV * LV * kGroup;
   int64_t k0 = (int64_t)w * kGroup;
-  if (k0 < K) {
+  if constexpr (LV > 1) {
+    // Slices in bit-reversed order, so that each pair the tree adds is complete before the next begins: level
+    // d of part holds a finished left half of 2^d slices. Empty slices are added as the zeros they are.
+    constexpr int LOG = LV == 4 ? 2 : 4;
+    static_assert(LV == 1 << LOG && NB == 1, "four or sixteen slices of one product");
+    f32x4 part[LOG][MF][CF], pcomp[LOG][F32 ? MF : 1][F32 ? CF : 1];
+    auto slice_k = [&](int i) { return (int64_t)(w + WV * (int)(__builtin_bitreverse32((unsigned)i) >> (32 - LOG))) * kGroup; };
+    auto finish = [&](int i) {
+      bool held = false;
+#pragma unroll
+      for (int d = 0; d < LOG; ++d) {
+        if (held) continue;
+        held = ((i >> d) & 1) == 0;  // uniform
+#pragma unroll
+        for (int x = 0; x < MF; ++x)
+#pragma unroll
+          for (int c = 0; c < CF; ++c) {
+            f32x4& s = part[d][x][c];
+            f32x4& sc = pcomp[d][F32 ? x : 0][F32 ? c : 0];
+            f32x4& ac = comp[0][F32 ? x : 0][F32 ? c : 0];
+            if (held) {
+              s = acc[0][x][c];
+              acc[0][x][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+              if constexpr (F32) {
+                sc = ac;
+                ac = f32x4{0.f, 0.f, 0.f, 0.f};
+              }
+            } else {
+              add(s, sc, acc[0][x][c], ac);
+              acc[0][x][c] = s;
+              if constexpr (F32) ac = sc;
+            }
+          }
+      }
+    };
+    struct At {
+      int i;
+      int64_t k;
+    };
+    auto settle = [&](At a) {  // the first group at or after a
+      while (a.k >= K) {
+        if (++a.i == LV) break;
+        a.k = slice_k(a.i);
+      }
+      return a;
+    };
+    int done = 0;
+    At at = settle(At{0, slice_k(0)});
+    if (at.i < LV) {
+      Group x0, x1;
+      load((int)at.k, x0);
+      while (true) {
+        At nx = settle(At{at.i, at.k + kStride});
+        if (nx.i < LV) load((int)nx.k, x1);
+        for (; done < at.i; ++done) finish(done);
+        compute(x0);
+        at = nx;
+        if (at.i == LV) break;
+        nx = settle(At{at.i, at.k + kStride});
+        if (nx.i < LV) load((int)nx.k, x0);
+        for (; done < at.i; ++done) finish(done);
+        compute(x1);
+        at = nx;
+        if (at.i == LV) break;
+      }
+    }
+    if (K > WV * kGroup)  // else each wave has one slice, and the others' zeros change nothing
+      for (; done < LV; ++done) finish(done);
+  } else if (k0 < K) {
     Group x0, x1;
     load((int)k0, x0);
     while (true) {
@@ -257,14 +339,8 @@ __global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typen
 #pragma unroll
           for (int c = 0; c < CF; ++c) {
             const int f = (b * MF + i) * CF + c;
-            const f32x4 o = slot[f * kParts * 64];
-            if constexpr (F32) {
-              const f32x4 s = acc[b][i][c], t = s + o, z = t - s;
-              comp[b][i][c] += slot[(f * kParts + 1) * 64] + ((s - (t - z)) + (o - z));
-              acc[b][i][c] = t;
-            } else {
-              acc[b][i][c] += o;
-            }
+            if constexpr (F32) add(acc[b][i][c], comp[b][i][c], slot[f * kParts * 64], slot[(f * kParts + 1) * 64]);
+            else add(acc[b][i][c], comp[0][0][0], slot[f * kParts * 64], comp[0][0][0]);
           }
     }
     __syncthreads();
@@ -331,11 +407,11 @@ __global__ __launch_bounds__(WV* kWave, small_occupancy(WV, MF, BT, sizeof(typen
   }
 }
 
-template <typename T, bool BT, int NB, int EPI, int MF, int CF, int WV, int U>
+template <typename T, bool BT, int NB, int EPI, int MF, int CF, int WV, int U, int LV = 1>
 static void launch_small_cfg(const void* A, const void* B0, const void* B1, void* C, int M, int N, int K, int64_t lda,
                              int64_t ldb, int64_t ldc, hipStream_t s, const EpiArgs& ep) {
   using S = typename T::S;
-  gemm_small<T, BT, NB, EPI, MF, CF, WV, U><<<dim3((unsigned)cdiv(N, 16 * CF), (unsigned)cdiv(M, 16 * MF), ep.batch), WV * kWave, 0, s>>>(
+  gemm_small<T, BT, NB, EPI, MF, CF, WV, LV, U><<<dim3((unsigned)cdiv(N, 16 * CF), (unsigned)cdiv(M, 16 * MF), ep.batch), WV * kWave, 0, s>>>(
       (const S*)A, (const S*)B0, (const S*)B1, (S*)C, M, N, K, lda, ldb, ldc, ep);
 }
 
@@ -345,6 +421,28 @@ int launch_gemm_small(const void* A, const void* B0, const void* B1, void* C, in
 #define AK_SM(BT, MF, CF, WV, U) \
   launch_small_cfg<T, BT, NB, EPI, MF, CF, WV, U>(A, B0, B1, C, (int)M, (int)N, (int)K, lda, ldb, ldc, s, ep)
   constexpr bool F32 = sizeof(typename T::S) == 4;
+  if constexpr (NB == 1 && EPI == kEpiStore) {
+    // A batch whose blocks pass the chip: four slices a wave on wider tiles, with the same sums (us, as one
+    // product / so: f16 nt 16 x 128 x 512, 64 items 8.1 / 6.9, 512 items 40 / 19; nn 1 x 4096 x 4096, 8 items 92 / 52;
+    // f32 nt 32 x 512 x 64, 64 items 20 / 16, 512 items 132 / 91). Not where that was no faster: f32 nt of few
+    // rows and much k (8 x 768 x 768, 32 items 20 / 24), nn in groups of one k-step (32 x 3000 x 1000, 8 items 33 / 38).
+    const int64_t blocks = N <= 4096 ? small_blocks(M, N, bt) * ep.batch : 0;
+    const bool k64 = small_k64(M, N, bt);
+    if (ep.batch > 1 && (F32 ? blocks > (bt ? 768 : 512) && !(bt && M <= 16 && K > 256) : blocks > 256 && (bt || k64))) {
+#define AK_SMB(MF, CF, U)                                                                                             \
+  if (bt) launch_small_cfg<T, true, 1, EPI, MF, CF, 4, U, 4>(A, B0, B1, C, (int)M, (int)N, (int)K, lda, ldb, ldc, s, ep); \
+  else launch_small_cfg<T, false, 1, EPI, MF, CF, 4, U, 4>(A, B0, B1, C, (int)M, (int)N, (int)K, lda, ldb, ldc, s, ep)
+      if (M <= 16) {
+        AK_SMB(1, 4, 2);
+      } else if (k64) {
+        AK_SMB(2, 2, 2);
+      } else {
+        AK_SMB(2, 2, 1);
+      }
+#undef AK_SMB
+      return record_launch();
+    }
+  }
   // Columns per block: few while N gives the chip few blocks (each block then walks K on 16 waves),
   // more for wide N, where the rows of A, re-read by every block, would cost as much as B.
   if (bt) {

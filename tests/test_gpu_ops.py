@@ -370,6 +370,25 @@ def test_batched_few_rows_of_any_stride(gpu, M, N, K, pad_a, pad_b):
                 assert torch.equal(out[z], host._gemm(A[z], B[z])), (z, M, N, K, pad_a, pad_b, dt)
 
 
+@pytest.mark.parametrize("Z,M,N,K", [(70, 16, 128, 512), (300, 1, 40, 1000), (8, 1, 4096, 4096), (70, 64, 64, 576), (5, 64, 1536, 2048),
+                                     (140, 64, 64, 576), (90, 50, 72, 2112), (12, 33, 1104, 2112), (12, 40, 1101, 77), (200, 20, 70, 8),
+                                     (9, 64, 4096, 2049)])
+@pytest.mark.parametrize("pad_a,pad_b", [(0, 0), (1, 3), (8, 0)])
+def test_batched_few_rows_past_the_chip(gpu, Z, M, N, K, pad_a, pad_b):
+    """Batches whose items' blocks together pass the chip run on four slices a wave or, f16 / bf16 of more than 16
+    rows, on tiles (LDS-DMA and register-staged, groups of 32 and 64 k), in gemm_small's order of the sums: fewer
+    groups than its 16 slices, more, and a ragged last one; each item equals its 2-D product bit for bit."""
+    from autokernel_amd.kernels import host
+    g = torch.Generator().manual_seed(M + N + K + pad_a)
+    for dt in (torch.float16, torch.bfloat16, torch.float32):
+        A = torch.randn(Z * (M * K + pad_a), generator=g).to(dt).to(gpu).as_strided((Z, M, K), (M * K + pad_a, K, 1))
+        Bf = torch.randn(Z * (K * N + pad_b), generator=g).to(dt).to(gpu)
+        for B in (Bf.as_strided((Z, N, K), (K * N + pad_b, K, 1)).transpose(1, 2), Bf.as_strided((Z, K, N), (K * N + pad_b, N, 1))):
+            out = kernels.get("matmul")(A, B)
+            for z in {*range(0, Z, 1 + Z // 20), Z - 1}:
+                assert torch.equal(out[z], host._gemm(A[z], B[z])), (z, dt, B.stride())
+
+
 @pytest.mark.parametrize("dt,K", [(torch.float16, 8), (torch.float16, 7), (torch.float32, 4)], ids=["f16", "f16 odd", "f32"])
 def test_matmul_few_rows_of_many_columns(gpu, dt, K):
     """2^28 columns against one row: gemm_small's 16 work-items per column would pass a grid's 2^32, so
