@@ -15,6 +15,13 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kLoopThreads = 256;
 constexpr int kWidestRow = 65536;  // elements of a row cached in registers (1024 lanes of 64)
+template <typename T, int L, int VPT, bool ANY>
+constexpr bool kWidest = ANY && L * VPT * T::kVec == kWidestRow;
+// whether the 16-byte pieces of a row this wide may be more than the widest kernel's lanes hold
+template <typename T>
+inline bool pieces_pass(int64_t cols) {
+  return cdiv(cols + T::kVec - 1, T::kVec) > kWidestRow / T::kVec;
+}
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -241,7 +248,9 @@ static int launch_layernorm(const void* x, const void* w, const void* b, void* y
 // =============================================================================================
 // Softmax over the last dim (reference.py:15-17): fp32 max, exp and sum, one rounding.
 // =============================================================================================
-template <typename T, int L, int VPT, bool ANY>
+// HEAD (also of ce_rows): unaligned rows of a width whose pieces may pass what the lanes hold; the others do
+// without the elements it leaves at the row's start (softmax f16 [4096, 50257] 158.9 us with them, 156.3).
+template <typename T, int L, int VPT, bool ANY, bool HEAD>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
     const typename T::S* __restrict__ x, typename T::S* __restrict__ y, int64_t rows, int cols, int nt_out) {
   using G = RowGeom<L>;
@@ -250,9 +259,8 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void softmax_rows(
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  constexpr bool kHead = ANY && L * VPT * T::kVec == kWidestRow;
-  const RowShape<T, ANY, kHead> sh(x + row * cols, cols, active, L * VPT);
-  const bool has_head = kHead && gl < sh.head();
+  const RowShape<T, ANY, HEAD> sh(x + row * cols, cols, active, L * VPT);
+  const bool has_head = HEAD && gl < sh.head();
   R r;
   r.load(x + row * cols, sh, gl);
   float h = has_head ? T::to_f(x[row * cols + gl]) : -INFINITY, m = h;
@@ -421,7 +429,9 @@ static int launch_softmax(const void* x, void* y, int64_t rows, int64_t cols, hi
   if (plan_row_cols(rows, cols, T::kVec, any, &plan)) {
     AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-      launch_timed(softmax_rows<T, L, VPT, ANY>, grid, dim3(RowGeom<L>::kThreads), 0, s, xp, yp, rows, (int)cols, nt_out);
+      auto run = [&](auto kernel) { launch_timed(kernel, grid, dim3(RowGeom<L>::kThreads), 0, s, xp, yp, rows, (int)cols, nt_out); };
+      if (kWidest<T, L, VPT, ANY> && pieces_pass<T>(cols)) run(softmax_rows<T, L, VPT, ANY, kWidest<T, L, VPT, ANY>>);
+      else run(softmax_rows<T, L, VPT, ANY, false>);
     }));
   } else if (cols >= T::kVec) {
     launch_timed(softmax_stream<T>, dim3((unsigned)rows), dim3(kLoopThreads), 0, s, xp, yp, (int)cols);
@@ -459,7 +469,7 @@ __device__ __forceinline__ float ce_row_loss_b2(const typename T::S* xr, int64_t
   return -lp;
 }
 
-template <typename T, int L, int VPT, bool ANY>
+template <typename T, int L, int VPT, bool ANY, bool HEAD>
 __global__ __launch_bounds__(RowGeom<L>::kThreads) void ce_rows(
     const typename T::S* __restrict__ x, const int64_t* __restrict__ tgt, float* __restrict__ loss,
     int64_t rows, int cols, int64_t ignore_index) {
@@ -469,9 +479,8 @@ __global__ __launch_bounds__(RowGeom<L>::kThreads) void ce_rows(
   const int gl = G::lane_in_row();
   const int64_t row = (int64_t)blockIdx.x * G::kRowsPerBlock + G::group();
   const bool active = row < rows;
-  constexpr bool kHead = ANY && L * VPT * T::kVec == kWidestRow;
-  const RowShape<T, ANY, kHead> sh(x + row * cols, cols, active, L * VPT);
-  const bool has_head = kHead && gl < sh.head();
+  const RowShape<T, ANY, HEAD> sh(x + row * cols, cols, active, L * VPT);
+  const bool has_head = HEAD && gl < sh.head();
   R r;
   r.load(x + row * cols, sh, gl);
   const float h = has_head ? T::to_f(x[row * cols + gl]) : -INFINITY;
@@ -568,7 +577,10 @@ static int launch_ce(const void* logits, const int64_t* tgt, float* loss, void* 
   if (!handled && planned && !stream) {
     AK_ANY_SWITCH(any, AK_ROW_SWITCH({
       const dim3 grid((unsigned)cdiv(rows, RowGeom<L>::kRowsPerBlock));
-      ce_rows<T, L, VPT, ANY><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, tgt, loss, rows, (int)vocab, ignore_index);
+      if (kWidest<T, L, VPT, ANY> && pieces_pass<T>(vocab))
+        ce_rows<T, L, VPT, ANY, kWidest<T, L, VPT, ANY>><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, tgt, loss, rows, (int)vocab, ignore_index);
+      else
+        ce_rows<T, L, VPT, ANY, false><<<grid, RowGeom<L>::kThreads, 0, s>>>(xp, tgt, loss, rows, (int)vocab, ignore_index);
     }));
   } else if (!handled && vocab >= T::kVec) {
     ce_stream<T><<<(unsigned)rows, kLoopThreads, 0, s>>>(xp, tgt, loss, (int)vocab, ignore_index);
