@@ -69,23 +69,26 @@ __device__ __forceinline__ u32x4 load_kchunk(const uint16_t* __restrict__ p, int
 // gemm_small's order of the sums (N <= 4096), for tiles of a batch of such products: slice i is k-groups i,
 // i + 16, ..., and the slices' sums are added as a tree over 16 waves adds them. With the slices visited in
 // bit-reversed order each pair of the tree is complete before the next begins, so four held tiles are enough.
+// Fewer groups than slices leave the upper slices empty: only the tree's levels below those are walked.
 struct SliceWalk {
-  int g = 0, i = 0;  // group, position of its slice (16: past the end)
-  __device__ __forceinline__ void step(int groups) {
-    for (g += 16; g >= groups && i < 16;) {
+  int groups, levels, g = 0, i = 0;  // i: position of g's slice (2^levels: past the end)
+  __device__ __forceinline__ explicit SliceWalk(int n) : groups(n), levels(n > 8 ? 4 : n > 4 ? 3 : n > 2 ? 2 : n > 1 ? 1 : 0) {}
+  __device__ __forceinline__ bool done() const { return i >> levels; }
+  __device__ __forceinline__ void step() {
+    for (g += 16; g >= groups && !done();) {
       ++i;
-      g = (int)(__builtin_bitreverse32((unsigned)i) >> 28);
+      g = (int)((__builtin_bitreverse32((unsigned)i) >> 1) >> (31 - levels));
     }
   }
 };
 // The slice at position i is in acc: hold it (acc starts the next) or add it to the held left halves it ends.
-// Level d of part holds 2^d slices. (In LDS, or with the walk unrolled, the tiles were slower.)
+// Level d of part holds 2^d slices. (With part in LDS, or with the walk unrolled, the tiles were slower.)
 template <int FM, int FN>
-__device__ __forceinline__ void end_slice(int i, f32x4 (&part)[4][FM][FN], f32x4 (&acc)[FM][FN]) {
+__device__ __forceinline__ void end_slice(int i, int levels, f32x4 (&part)[4][FM][FN], f32x4 (&acc)[FM][FN]) {
   bool held = false;
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
-    if (held) continue;
+    if (held || d >= levels) continue;
     held = ((i >> d) & 1) == 0;  // uniform
 #pragma unroll
     for (int x = 0; x < FM; ++x)
@@ -230,10 +233,10 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
   const int groups = SL ? (K + SL - 1) / (SL ? SL : 1) : 0;
   const int KT = SL == 32 ? (groups + 1) / 2 : (K + kBK - 1) / kBK;
   f32x4 part[4][SL ? FM : 1][SL ? FN : 1];
-  SliceWalk fetch, use;
+  SliceWalk fetch(groups), use(groups);
   auto take = [&]() {  // the next group's k; past the last one K, whose loads are zeros
-    const int k = fetch.i < 16 ? fetch.g * SL : K;
-    fetch.step(groups);
+    const int k = fetch.done() ? K : fetch.g * SL;
+    fetch.step();
     return k;
   };
   auto load_tile = [&](int kt) {
@@ -277,8 +280,8 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_mfma(
       if constexpr (SL != 0) {
         if (SL == 32 || s == 1) {
           int i = use.i;
-          use.step(groups);
-          for (; i < use.i; ++i) end_slice<FM, FN>(i, part, acc[0]);
+          use.step();
+          for (; i < use.i; ++i) end_slice<FM, FN>(i, use.levels, part, acc[0]);
         }
       }
     }
@@ -392,13 +395,13 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
 
   const int KT = K / BKD;
   f32x4 part[4][SL ? FM : 1][SL ? FN : 1];
-  SliceWalk fetch, use;
+  SliceWalk fetch(KT), use(KT);
   auto issue = [&](int kt, uint16_t* sp) {
     if constexpr (SL) {  // issues come in the tiles' order; past the end the last one again
       kt = fetch.g;
       SliceWalk n = fetch;
-      n.step(KT);
-      if (n.i < 16) fetch = n;
+      n.step();
+      if (!n.done()) fetch = n;
     }
     const uint32_t kb = 2u * (uint32_t)(kt * BKD);
     const uint32_t kbb = BKN ? (uint32_t)kt * kb_step_b : kb;
@@ -474,20 +477,36 @@ __device__ __forceinline__ void gemm_dma_ns_kloop(
   dma_barrier<(NS - 1) * INS>();
   load_a(s0, 0, 0, FM);
   load_b(s0, 0, fb);
-  for (int kt = 0; kt < KT; kt += NS) {
+  if constexpr (SL) {
+    static_assert(NB == 1 && NS == 4, "slices of one product, in four stages");
+    constexpr int kStage = (BM + BN) * BKD;
+    // Not unrolled over the stages (which are one array): the longer code cost more to fetch than it saved (us,
+    // unrolled / so: 128 x [64 x 64 x 512] 10.3 / 8.5, 256 x [32 x 1024 x 512] 80 / 73; 128 x [64 x 1024 x 1024] 73 / 76).
+#pragma unroll 1
+    for (int t = 0; t < KT; ++t) {
+      uint16_t* const cur = s0 + (t & 3) * kStage;
+      uint16_t* const nxt = s0 + ((t + 1) & 3) * kStage;
 #pragma unroll
-    for (int u = 0; u < NS; ++u) {
-      const int t = kt + u;
-      if (t < KT) {  // uniform over the block
+      for (int s = 0; s < STEPS; ++s) {
+        if (s + 1 < STEPS) kstep(cur, s + 1, false, cur, 0);
+        else kstep(nxt, 0, true, cur, 0);
+      }
+      int i = use.i;
+      use.step();
+#pragma unroll 1
+      for (; i < use.i; ++i) end_slice<FM, FN>(i, use.levels, part, acc[0]);
+    }
+  } else {
+    for (int kt = 0; kt < KT; kt += NS) {
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-          if (s + 1 < STEPS) kstep(st[u], s + 1, false, st[u], 0);
-          else kstep(st[(u + 1) % NS], 0, true, st[u], min(t + NS, KT - 1));
-        }
-        if constexpr (SL) {
-          int i = use.i;
-          use.step(KT);
-          for (; i < use.i; ++i) end_slice<FM, FN>(i, part, acc[0]);
+      for (int u = 0; u < NS; ++u) {
+        const int t = kt + u;
+        if (t < KT) {  // uniform over the block
+#pragma unroll
+          for (int s = 0; s < STEPS; ++s) {
+            if (s + 1 < STEPS) kstep(st[u], s + 1, false, st[u], 0);
+            else kstep(st[(u + 1) % NS], 0, true, st[u], min(t + NS, KT - 1));
+          }
         }
       }
     }
@@ -557,10 +576,13 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC* WM* WN / 4) void gemm_dma(
   static_assert(4 * (A_INS + NB * B_INS) < 64, "outstanding DMA fits vmcnt");
   static_assert(FM % 2 == 0, "two MFMA halves per k-step");
   constexpr int kStage = (BM + NB * BN) * BKD;  // elements per stage
-  __shared__ __attribute__((aligned(1024))) uint16_t sS0[kStage];
-  __shared__ __attribute__((aligned(1024))) uint16_t sS1[kStage];
-  __shared__ __attribute__((aligned(1024))) uint16_t sS2[NS > 2 ? kStage : 1];
-  __shared__ __attribute__((aligned(1024))) uint16_t sS3[NS > 3 ? kStage : 1];
+  __shared__ __attribute__((aligned(1024))) uint16_t sS0[SL ? NS * kStage : kStage];
+  __shared__ __attribute__((aligned(1024))) uint16_t sS1s[SL ? 1 : kStage];
+  __shared__ __attribute__((aligned(1024))) uint16_t sS2s[!SL && NS > 2 ? kStage : 1];
+  __shared__ __attribute__((aligned(1024))) uint16_t sS3s[!SL && NS > 3 ? kStage : 1];
+  uint16_t* const sS1 = SL ? sS0 + kStage : sS1s;
+  uint16_t* const sS2 = SL ? sS0 + 2 * kStage : sS2s;
+  uint16_t* const sS3 = SL ? sS0 + 3 * kStage : sS3s;
 
   if constexpr (EPI == kEpiPartial) {
     const int z = (int)blockIdx.y;  // K slice
@@ -859,8 +881,8 @@ static void launch_gemm_dma(const void* A, const void* B0, const void* B1, void*
 
 // A batch of products that each take gemm_small, summed in its order by tiles: past 512 blocks of 32 x 32 the
 // tiles, which share their operands' loads, are the faster form (us, a block's 16 waves / four slices a wave / these:
-// f16 nt 64 x 64 x 512, 64 items 12.4 / 7.5 / 10.2, 512 items 76 / 27 / 17; 64 x 1024 x 1024, 4 items 15 / 8 / 13, 128 items 425 /
-// 137 / 72; nn 32 x 3000 x 1000, 8 items 33 / 38 / 26). dma: the LDS-DMA kernel reads them; vec: 16-byte loads do.
+// f16 nt 64 x 64 x 512, 128 items 22 / 10 / 8.5, 512 items 76 / 27 / 16; 64 x 1024 x 1024, 4 items 15 / 8 / 13, 128 items 425 /
+// 137 / 76; nn 32 x 3000 x 1000, 8 items 33 / 38 / 24). dma: the LDS-DMA kernel reads them; vec: 16-byte loads do.
 template <typename T>
 static int launch_gemm_slices(const void* A, const void* B, void* C, int M, int N, int K, int64_t lda, int64_t ldb,
                               int64_t ldc, bool bt, bool dma, bool vec, hipStream_t s, const EpiArgs& ep) {
