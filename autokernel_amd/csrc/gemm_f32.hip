@@ -16,7 +16,7 @@
 //     fp32 sum of K = 8192 is 4.9e-4 off).
 // The order of the additions depends on k alone, so every tile size and layout gives the same bits.
 //
-// Measured, f32 2048^3: 306 -> 172 us (4-byte loads and LDS reads before: 56 TFLOP/s), 4096^3 98-104
+// Measured, f32 2048^3: 306 -> 173 us (4-byte loads and LDS reads before: 56 TFLOP/s), 4096^3 98-104
 // TFLOP/s; 1024^3, whose 64 tiles of 128 x 128 left most CUs idle, 154 -> 39 us on 64 x 64 tiles.
 // Without the Kahan steps (a timing-only build) 2048^3 takes 17 % less. The error against 64 bits is
 // 7.9e-8 (8.1e-8 before), a plain fp32 sum's 8.1e-7.

@@ -486,8 +486,8 @@ def _assert_same_non_finite(out, want, what):
 @pytest.mark.parametrize("K", [1, 8, 16, 17, 32, 40, 48, 64, 1000])
 def test_f32_tiles_keep_infinities(gpu, M, N, K):
     """fp32 products and gate/up (64 and 128 tiles) with infinities, NaN and overflowing sums at every
-    place in a k-tile give what a plain sum gives: the compensation of an infinite total is bounded,
-    so that the steps after it, those on a tile's zero padding included, leave the total alone."""
+    place in a k-tile give what a plain sum gives, also where steps follow the one that made a total
+    infinite (those on a tile's zero padding included): a block that ends with a NaN adds again, plainly."""
     from autokernel_amd.kernels import _ops, host
     A = _non_finite_rows(M, K)
     for bt in (True, False):
@@ -1053,8 +1053,8 @@ WIDE_TOL = {torch.float16: 1e-3, torch.bfloat16: 2e-3, torch.float32: 1e-5}
 @pytest.mark.parametrize("cols", [4097, 16383, 16385, 50257, 65535, 65537])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
 def test_softmax_ce_wide_odd_rows(gpu, cols, dtype):
-    """Widths that do not vectorise, on each side of the register-cached wide-row kernels' limits
-    (4096 < cols <= 16 * 1024 and <= 64 * 1024; 65537 stays on the looped kernel): softmax and
+    """Widths that are no multiple of a vector, on each side of what a block of 1024 lanes caches in
+    registers (65536 columns; 65537 streams): softmax and
     cross-entropy against the oracle, with a row holding -inf entries, a row of large values and a
     constant row, and bitwise-equal reruns."""
     g = torch.Generator().manual_seed(cols)
